@@ -449,8 +449,9 @@ static uint64_t carve_scratch(pg_engine* e, char* b, uint64_t bodies, uint64_t n
     const uint64_t o_tp = take((node_tiles + 2) * sizeof(Sum4));
     const uint64_t o_lf = take((node_tiles + 2) * kTopSlots * 4);
     const uint64_t o_dk = take(bodies * sizeof(DeepKey));
-    const uint64_t o_hot = take(nodes * sizeof(NodeHot));
-    const uint64_t o_span = take(nodes * sizeof(uint2)), o_lp = take(bodies * sizeof(double4));
+    // (one more entry than nodes: the walk's end of the array)
+    const uint64_t o_hot = take((nodes + 1) * sizeof(NodeHot));
+    const uint64_t o_span = take((nodes + 1) * sizeof(uint2)), o_lp = take(bodies * sizeof(double4));
     const uint64_t o_acc = take(bodies * 24);
     const uint64_t o_d0 = take(segs * sizeof(SegDesc)), o_d1 = take(segs * sizeof(SegDesc));
     const uint64_t o_so = take((segs + 1) * 8);
@@ -761,7 +762,8 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
     });
     launch(e, cap, "tree_scan", [&] {
         k_tree_scan<<<1 + kTopSlots, kScanThreads, 0, st>>>(e->tile_tot, e->tile_base, tiles,
-                                                             e->lvl_first, e->first_node, total);
+                                                             e->lvl_first, e->first_node, total,
+                                                             e->node_span, e->cap_nodes);
     });
     launch(e, cap, "nodes", [&] {
         k_nodes<DIM><<<tiles, kNodeThreads, 0, st>>>(
@@ -1769,16 +1771,7 @@ extern "C" int pg_sim_tree(pg_sim* s, int64_t* rec, double* fl, uint64_t cap, ui
         ++out;
     };
     for (uint64_t b = 0; b < n && out < cap; ++b) {
-        // the internal nodes that start at body b (shallowest first), then its leaf
-        for (; k < ni && span[k].x == b; ++k) {
-            const NodeHot& h = hot[k];
-            const int L = h.level();
-            put(L, L > 0 ? (int64_t)h.octant() : -1, -1, (int64_t)b, h.mass, h.mx, h.my, h.mz,
-                h.cx, h.cy, h.cz);
-        }
-        // the leaf's level, octant and centre: the reference's descent
-        // (octree.rs:160-215 / quadtree.rs:161-194) along the body's key, the
-        // same operations as the device's
+        // the body's leaf level and its path's octants, by its key's digits
         const int L = (int)lo[b] + (int)(fn[b + 1] - fn[b]);
         if (L > lmax && deep.empty()) {
             deep.resize(n);
@@ -1791,6 +1784,16 @@ extern "C" int pg_sim_tree(pg_sim* s, int64_t* rec, double* fl, uint64_t cap, ui
             const int t = l - lmax;
             return (uint32_t)((deep[b].w[t / wl] >> (dim * (wl - 1 - t % wl))) & mask);
         };
+        // the internal nodes that start at body b (shallowest first), then its leaf
+        for (; k < ni && span[k].x == b; ++k) {
+            const NodeHot& h = hot[k];
+            const int L = (int)(h.level2 / 2);
+            put(L, L > 0 ? (int64_t)digit(L - 1) : -1, -1, (int64_t)b, h.mass, h.mx, h.my, h.mz,
+                h.cx, h.cy, h.cz);
+        }
+        // the leaf's octant and centre: the reference's descent
+        // (octree.rs:160-215 / quadtree.rs:161-194) along the body's key, the
+        // same operations as the device's
         double ext = E, c[3] = {0.0, 0.0, 0.0};
         for (int l = 0; l < L; ++l) {
             const uint32_t o = digit(l);

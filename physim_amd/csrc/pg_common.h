@@ -112,17 +112,18 @@ struct SegState {
     uint32_t vperm;         // velocities must travel with the state (not yet derivable)
 };
 
-// Internal tree node record, one 64-byte line (what the walk reads per
-// visited node). Every field is a whole number of 32-bit words, so the walk
-// fetches a record through the scalar unit (which has no 16-bit loads).
+// Internal tree node record, one 64-byte line: what the walk's opening test
+// reads in the first half (fetched through the scalar unit), the source a body
+// that takes the node adds in the second (the form of a leaf's position
+// record). Skip and level are kept as the walk uses them: a byte offset into
+// the span array (8 bytes per node; times 8, into the records) and the
+// exponent of 4^level.
 struct NodeHot {
     double cx, cy, cz;      // geometric centre (reference rounding)
+    uint32_t skip8;         // 8 * index of the next internal node after this subtree
+    uint32_t level2;        // 2 * level
     double mx, my, mz;      // centre of mass
     double mass;
-    uint32_t skip;          // index of the next internal node after this subtree
-    uint32_t lvl_oct;       // level (bits 0-15), child index within the parent (bits 16-23)
-    __host__ __device__ int level() const { return (int)(lvl_oct & 0xFFFFu); }
-    __host__ __device__ uint32_t octant() const { return (lvl_oct >> 16) & 0xFFu; }
 };
 
 // Batch-wide counters reset at the start of every step.

@@ -21,16 +21,12 @@ __device__ __forceinline__ uint32_t f32_bits(float f) { return __float_as_uint(f
 // into the subnormal range), without relying on the compiler to see that.
 __device__ __forceinline__ double half(double x) { return x * 0.5; }
 
-// A uniform double copied into a vector register. The walk copies an item's
-// source (a node's centre of mass and mass, read through the scalar unit)
-// before it loads the next node record: the record then lands in the
-// registers it is carried in, and the pair term runs while the load is in
-// flight, instead of the compiler copying the new record over and waiting
-// for it first. (A move, not a load: nothing is in flight in it.)
-__device__ __forceinline__ double vcopy(double v) {
-    double r;
-    asm("v_mov_b64 %0, %1" : "=v"(r) : "s"(v));
-    return r;
+// v with lane `lane` (uniform) replaced by the uniform value x (v_writelane;
+// the compiler names no builtin for it, only the intrinsic).
+__device__ uint32_t writelane_u32(uint32_t x, uint32_t lane, uint32_t v) __asm(
+    "llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ uint32_t write_lane(uint32_t v, uint32_t x, uint32_t lane) {
+    return writelane_u32(x, lane, v);
 }
 
 __device__ __forceinline__ uint32_t uniform_u32(uint32_t v) {
@@ -137,20 +133,6 @@ template <int DIM>
 constexpr int kWordLevels = DIM == 3 ? 21 : 32;
 static_assert(21 + kDeepWords * 21 > kMaxLcp && 32 + kDeepWords * 32 > kMaxLcp,
               "a first word and the deep key resolve every level a prefix may reach");
-
-template <int DIM>
-__device__ __forceinline__ uint32_t deep_digit(const DeepKey& k, int t) {
-    constexpr int W = kWordLevels<DIM>;
-    return (uint32_t)((k.w[t / W] >> (DIM * (W - 1 - t % W))) & ((1u << DIM) - 1u));
-}
-
-// Octant digit taken at tree depth d (from level d to level d + 1).
-template <int DIM>
-__device__ __forceinline__ uint32_t key_digit(uint64_t key, const DeepKey& dk, int lmax, int d) {
-    const uint64_t dmask = (1u << DIM) - 1u;
-    return d < lmax ? (uint32_t)((key >> (DIM * (lmax - 1 - d))) & dmask)
-                    : deep_digit<DIM>(dk, d - lmax);
-}
 
 // Common prefix length, in levels, of two deep keys.
 template <int DIM>
@@ -2182,11 +2164,13 @@ __device__ __forceinline__ uint32_t block_inclusive_scan(uint32_t v, uint32_t* s
 }
 
 // Block 0: exclusive scan of the tile node totals into tile_base[0..tiles]
-// (tile_base[tiles] = all nodes) and first_node[total] = all nodes. Block
+// (tile_base[tiles] = all nodes) and first_node[total] = all nodes, and the
+// span past the last node (entry min(all, cap) of cap + 1). Block
 // 1 + L: suffix minimum over the tiles of lvl_first[., L], in place.
 __global__ __launch_bounds__(kScanThreads) void k_tree_scan(
     const uint32_t* __restrict__ tile_tot, uint32_t* __restrict__ tile_base, uint32_t tiles,
-    uint32_t* __restrict__ lvl_first, uint32_t* __restrict__ first_node, uint64_t total) {
+    uint32_t* __restrict__ lvl_first, uint32_t* __restrict__ first_node, uint64_t total,
+    uint2* __restrict__ node_span, uint64_t cap) {
     __shared__ uint32_t s_wave[kScanThreads / 64];
     // a thread's first kKeep values stay in registers between the scan's
     // two passes (up to kKeep * kScanThreads tiles: no second read)
@@ -2221,6 +2205,8 @@ __global__ __launch_bounds__(kScanThreads) void k_tree_scan(
         if (threadIdx.x == 0) {
             tile_base[tiles] = all;
             first_node[total] = all;
+            // the walk's end of the node array: a span that starts at no body
+            node_span[min((uint64_t)all, cap)] = make_uint2(~0u, ~0u);
         }
         return;
     }
@@ -2470,24 +2456,19 @@ static_assert(kNodeTile <= 1024 && kTopSlots <= 65, "queue entries: 10-bit bodie
 static_assert(kTopSlots * (kNodeTile / (kSmallNode + 1)) <= 2 * kNodeQueue && kTopSlots <= 65,
               "queue bound of the body-parallel build");
 
-// A node record as four 16-byte chunks: (cx, cy), (cz, mx), (my, mz),
-// (mass, skip, level | octant << 16), or as eight 8-byte words.
+// A node record as four 16-byte chunks: (cx, cy), (cz, 8 skip, 2 level),
+// (mx, my), (mz, mass).
 static_assert(sizeof(NodeHot) == 64, "one node record per 64-byte line");
-static_assert(offsetof(NodeHot, mass) == 48 && offsetof(NodeHot, skip) == 56 &&
-                  offsetof(NodeHot, lvl_oct) == 60,
+static_assert(offsetof(NodeHot, skip8) == 24 && offsetof(NodeHot, level2) == 28 &&
+                  offsetof(NodeHot, mx) == 32 && offsetof(NodeHot, mass) == 56,
               "chunk layout of a node record");
 __device__ __forceinline__ uint4 pack2(double a, double b) {
     const uint64_t x = f64_bits(a), y = f64_bits(b);
     return make_uint4((uint32_t)x, (uint32_t)(x >> 32), (uint32_t)y, (uint32_t)(y >> 32));
 }
-__device__ __forceinline__ uint2 pack1(double a) {
+__device__ __forceinline__ uint4 pack_skip(double a, uint32_t skip, uint32_t level) {
     const uint64_t x = f64_bits(a);
-    return make_uint2((uint32_t)x, (uint32_t)(x >> 32));
-}
-__device__ __forceinline__ uint4 pack_tail(double mass, uint32_t skip, uint32_t level,
-                                           uint32_t octant) {
-    const uint64_t x = f64_bits(mass);
-    return make_uint4((uint32_t)x, (uint32_t)(x >> 32), skip, level | (octant << 16));
+    return make_uint4((uint32_t)x, (uint32_t)(x >> 32), skip * 8u, level * 2u);
 }
 
 // Builds the tree's internal nodes and their masses and centres of mass,
@@ -2499,7 +2480,7 @@ __device__ __forceinline__ uint4 pack_tail(double mass, uint32_t skip, uint32_t 
 // The tile's bodies own the preorder range [tile_base[t], tile_base[t+1]) of
 // internal nodes (tile base + offsets within the tile, also written out as
 // first_node). Every internal node gets its geometric centre by the
-// reference's descent, its level, octant and skip (= first internal node of
+// reference's descent, its level and skip (= first internal node of
 // the body after its range) in its record, and its body range (first body,
 // body after the range) in node_span. A node's range end is found by a
 // galloping search over the staged keys (keys carry their segment, so no
@@ -2741,12 +2722,11 @@ __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6)
         return s_first[e];
     };
     // The record of internal node nd (level L, owned by local body li,
-    // geometric centre c, octant oct), and its body range. A tile-spanning
+    // geometric centre c), and its body range. A tile-spanning
     // node (the only one of its level that starts in the tile and leaves it)
     // gets zero mass here and its own from k_com_span; a larger internal
     // node is queued, its mass words written by the group pass.
-    auto emit = [&](uint32_t nd, uint32_t li, int L, double cx, double cy, double cz,
-                    uint32_t oct) {
+    auto emit = [&](uint32_t nd, uint32_t li, int L, double cx, double cy, double cz) {
         Sum4 c{0.0, 0.0, 0.0, 0.0};
         bool queued = false;
         uint64_t last;
@@ -2776,18 +2756,13 @@ __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6)
         }
         // first body and the body after the range (global sorted indices)
         node_span[nd] = make_uint2((uint32_t)(b0 + li), (uint32_t)(last + 1));
-        uint2* w = reinterpret_cast<uint2*>(hot + nd);
-        const uint4 tail = pack_tail(c.m, skip, (uint32_t)L, oct);
-        if (queued) {
-            reinterpret_cast<uint4*>(w)[0] = pack2(cx, cy);
-            w[2] = pack1(cz);
-            w[7] = make_uint2(tail.z, tail.w);
-        } else {
-            uint4* rec = reinterpret_cast<uint4*>(w);
-            rec[0] = pack2(cx, cy);
-            rec[1] = pack2(cz, c.x);
-            rec[2] = pack2(c.y, c.z);
-            rec[3] = tail;
+        uint4* rec = reinterpret_cast<uint4*>(hot + nd);
+        rec[0] = pack2(cx, cy);
+        // (a tree past the node capacity, an error, leaves the walk in range)
+        rec[1] = pack_skip(cz, (uint32_t)min((uint64_t)skip, cap), (uint32_t)L);
+        if (!queued) {
+            rec[2] = pack2(c.x, c.y);
+            rec[3] = pack2(c.z, c.m);
         }
     };
 
@@ -2799,8 +2774,7 @@ __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6)
         const int f = min(L, lt);
         double ext = s_path[f][0], cx = s_path[f][1], cy = s_path[f][2], cz = s_path[f][3];
         descend<DIM>(key, kx, lmax, f, L, ext, cx, cy, cz);
-        const uint32_t oct = L > 0 ? key_digit<DIM>(key, kx, lmax, L - 1) : 0u;
-        emit(nd, li, L, cx, cy, cz, oct);
+        emit(nd, li, L, cx, cy, cz);
     };
     if (node_par) {
         // one thread per internal node (listed in node order by the bodies:
@@ -2827,8 +2801,7 @@ __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6)
                 const int L = lo + k;
                 const uint64_t nd = (uint64_t)nbase + (uint64_t)k;
                 if (nd >= cap) break;  // reported above
-                const uint32_t oct = L > 0 ? key_digit<DIM>(key, kx, lmax, L - 1) : 0u;
-                emit((uint32_t)nd, li, L, cx, cy, cz, oct);
+                emit((uint32_t)nd, li, L, cx, cy, cz);
                 if (k + 1 < cnt) descend<DIM>(key, kx, lmax, L, L + 1, ext, cx, cy, cz);
             }
         }
@@ -2929,10 +2902,9 @@ __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6)
         }
         const Sum4 c = com_of(range_sum_row(s_bm, s_bx, s_by, s_bz, li, e));
         if ((threadIdx.x & 15u) == 0) {
-            uint2* w = reinterpret_cast<uint2*>(hot + nd);
-            w[3] = pack1(c.x);
-            reinterpret_cast<uint4*>(w)[2] = pack2(c.y, c.z);
-            w[6] = pack1(c.m);
+            uint4* rec = reinterpret_cast<uint4*>(hot + nd);
+            rec[2] = pack2(c.x, c.y);
+            rec[3] = pack2(c.z, c.m);
         }
     }
 }
@@ -3005,53 +2977,19 @@ struct Kahan3 {
     }
 };
 
-// The reference's opening test, `half_width / r < theta` with
-// r = sqrt(dx*dx + dy*dy + dz*dz) in FP64 (octree.rs:137-140), decided
-// exactly. An FP32 estimate hw * rsq(s) is within 3.3e-7 (relative) of the
-// exact quotient (conversions 6e-8 each, rsq 1.2e-7, product 6e-8), and the
-// FP64 quotient of the reference within 2.3e-16 of it, so outside a band of
-// 1e-6 * theta the estimate decides as the reference does. Inside the band,
-// or with operands outside FP32's normal range, the FP64 square root and
-// division decide.
-// Lanes for which `act` holds take the decision; the FP32 estimate is formed
-// for every lane and only the FP64 test (lanes inside the band) is behind a
-// branch, so the common path has no exec-mask handling.
-__device__ __forceinline__ bool accept_cell(double hw, double s, double theta, bool act) {
-    const bool inr = s > 1e-30 && s < 1e30 && hw > 1e-30 && hw < 1e30;
-    const float q = (float)hw * __builtin_amdgcn_rsqf((float)s);
-    const float t = (float)theta;
-    const float band = 1e-6f * fabsf(t);
-    const bool yes = q < t - band, no = q > t + band;
-    bool take = yes;
-    if (act && !(inr && (yes || no))) take = hw / sqrt(s) < theta;
-    return take;
-}
-
-
-// Pair acceleration on body a from (b, mb), mixed precision: the separation
-// b - a is taken in FP64 and rounded once; |F|/m_a = mb / (s + e) along the
-// unsoftened direction (astro/src/lib.rs:84-113, with m_a cancelled). Where
-// `use` is false (or the separation rounds to zero) the term is zero; where
-// `take` is false the lane takes nothing from this source and its sums are
-// left as they were (not even a zero is added: a compensated add of zero
-// moves the sum's bits). Both by selects rather than branches: no exec-mask
-// handling in the walk's loop.
-__device__ __forceinline__ void pair_mixed(double ax, double ay, double az, double bx, double by,
-                                              double bz, double mb, float ef, Kahan3& acc,
-                                              bool take, bool use) {
+// Pair acceleration on body a from (b, mb), mixed precision, as the terms of
+// a compensated sum: the separation b - a is taken in FP64 and rounded once;
+// |F|/m_a = mb / (s + e) along the unsoftened direction
+// (astro/src/lib.rs:84-113, with m_a cancelled). A body's own position, which
+// the reference skips, rounds to a zero separation and gives zero (adding
+// that zero is a step of the compensated sum like any other).
+__device__ __forceinline__ float3 pair_mixed(double ax, double ay, double az, double bx, double by,
+                                             double bz, float mb, float ef) {
     const float fx = (float)(bx - ax), fy = (float)(by - ay), fz = (float)(bz - az);
     const float s = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
-    const float w = use && s > 0.0f
-                        ? (float)mb * __builtin_amdgcn_rsqf(s) * __builtin_amdgcn_rcpf(s + ef)
-                        : 0.0f;
-    Kahan3 n = acc;
-    n.add(fx * w, fy * w, fz * w);
-    acc.sx = take ? n.sx : acc.sx;
-    acc.sy = take ? n.sy : acc.sy;
-    acc.sz = take ? n.sz : acc.sz;
-    acc.cx = take ? n.cx : acc.cx;
-    acc.cy = take ? n.cy : acc.cy;
-    acc.cz = take ? n.cz : acc.cz;
+    const float w =
+        s > 0.0f ? mb * __builtin_amdgcn_rsqf(s) * __builtin_amdgcn_rcpf(s + ef) : 0.0f;
+    return make_float3(fx * w, fy * w, fz * w);
 }
 
 // Pair force on a from b exactly as astro/src/lib.rs:84-113 computes it (FP64,
@@ -3067,35 +3005,273 @@ __device__ __forceinline__ void pair_fp64(double ax, double ay, double az, doubl
     f[2] += r2 * 1.0 * am * bm / re;
 }
 
-// Barnes-Hut walk of one sorted body per lane, wave-coherent and stackless:
-// the wave steps through the preorder node array together (one node address
-// per wave, so node loads are scalar); each lane applies the reference's own
-// opening test (octree.rs:137-157: accept iff half_width / |x - centre| <
-// theta, at every node, own cell included) and skips an accepted subtree
-// through its skip index; the wave descends into a node iff some lane opened
-// it. Then the Stormer update (verlet.rs:24-82) in place on the permuted
-// state, or the acceleration into acc_out (upload order) without it.
-// (a waves-per-EU hint of 6: the three records in flight fit the scalar
-// registers with almost no spills, at seven waves per SIMD, eight for the
-// mixed walk without the near-field test; a hint of 8 spilled 34 scalar
-// registers into vector lanes, whose reloads are VALU instructions in every
-// iteration and cost more than the eighth wave hid)
+// Barnes-Hut walk of one sorted body per lane, in two alternating phases per
+// wave.
+//
+// (1) The wave steps through the preorder node array together (one node
+// address per wave, so node loads are scalar), stackless: each lane applies
+// the reference's own opening test (octree.rs:137-157: accept iff half_width
+// / |x - centre| < theta, at every node, own cell included) and skips an
+// accepted subtree through its skip index; the wave descends into a node iff
+// some lane opened it. An item (node or leaf) that some lane takes gets a
+// number, and each lane that takes it writes that number to its own list in
+// LDS. (2) After kWalkItems items their sources (centre of mass and mass, or
+// a leaf's body) are fetched to LDS, one per lane, and every lane adds its
+// own list's terms in order.
+//
+// Of the items a wave visits a body takes less than half (at theta 0.5 about
+// 410 of 1,050 over 262,144 bodies, the longest list of a wave 450), so the
+// pair terms, most of the vector instructions, are formed about 650 times
+// (the lists' maxima over all chunks) instead of once per item. The terms and
+// their order per body are those of a plain preorder walk. What bounds it:
+// phase (1) is three quarters of the time, bound by scalar issue (one
+// instruction a clock for a CU's four SIMDs) and, with few waves, by the
+// latency of each next record; walk_items is written out for both. Chunks of
+// 64: of 32 or 48 leave LDS for eight waves a SIMD instead of six, but their
+// lists' maxima and fetches cost more (386 against 414 and 396 us below); of
+// 128, 3% fewer terms but half the waves. Against the walk with one phase (a
+// term per item, six selects to keep it): 262,144-body Plummer sphere at theta
+// 0.5 645 -> 390 us, 1M-body collision with a near field 2470 -> 1550,
+// 65,539-body cube at theta 0.7 in FP64 193 -> 118, 1M-body cube at theta 1.5
+// (one or two items a wave) 41.4 and 41.5.
+constexpr uint32_t kWalkItems = 64;  // items per chunk: one source fetch per lane
+constexpr uint32_t kWalkStride = 17; // words per lane's list of byte entries: an odd LDS stride
+static_assert(kWalkItems == 64 && 4 * kWalkStride > kWalkItems && kWalkStride % 2 == 1,
+              "a lane lists each item of a chunk at most once, and writes one entry past them");
+
 // Levels below a body's leaf at which its near field still opens cells.
-constexpr int kNearLevels = 2;
+constexpr uint32_t kNearLevels = 2;
+
+// The lanes of the wave for which a comparison holds, and the inverse: the
+// lane predicate of a mask. (Masks combined as scalar words stay in the scalar
+// unit; a ballot of a combined predicate takes two more vector instructions.)
+__device__ __forceinline__ uint64_t lanes_where(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ bool lane_in(uint64_t mask) __asm("llvm.amdgcn.inverse.ballot.i64");
+
+// A uniform double in scalar registers (left to itself the compiler keeps the
+// result of uniform FP64 arithmetic in vector registers).
+__device__ __forceinline__ double scalar_f64(double v) {
+    uint32_t a = (uint32_t)f64_bits(v), c = (uint32_t)(f64_bits(v) >> 32);
+    asm volatile("" : "+v"(a), "+v"(c));
+    return __hiloint2double((int)uniform_u32(c), (int)uniform_u32(a));
+}
+
+// The LDS byte address of a pointer to shared memory.
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
+// Orders a wave's LDS writes before its lanes' later reads of them (and the
+// reverse): one wave, so no barrier.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One wave's place in phase (1) of the walk. Nodes are named by their byte
+// offset into the span array (8 bytes each).
+struct WalkState {
+    uint32_t b, k8;             // the next item (uniform)
+    uint32_t items;             // items of this chunk (uniform)
+    uint64_t leaf;              // bit i: item i is a leaf (uniform)
+    uint32_t it;                // lane i: item i's node or body
+    uint32_t entry;             // LDS address of the end of the lane's list
+    uint32_t skip_until;        // the lane skips the items of the bodies below this
+    double d[3], q;             // scratch
+};
+// What it needs throughout (uniform; the near field's per lane).
+struct WalkConst {
+    const NodeHot* hot;
+    const uint2* span;
+    uint32_t bend;
+    double t_yes, t_no;
+    double x, y, z;
+    // near field: 2 * level bounds of the wave's lanes outside which no cell
+    // is tested; per lane: extent, margin, 2 * first and last level tested
+    uint32_t near_lo, near_hi;
+    double extent, margin;
+    uint32_t lane_lo, lane_hi;
+};
+
+// Phase (1)'s loop. A CU issues one scalar instruction a clock for its four
+// SIMDs, and as the compiler lays this loop out (60 scalar instructions for a
+// node that some lanes take) that, with the wait for each next record, is
+// what bounds the walk; written out it takes 16 scalar and 16 vector ones.
+// Two sets of scalar registers hold a node's record half and span (s64-s73,
+// s76-s85); the record after a node's subtree, where three of four nodes go
+// next, loads into the other set while the node is tested. Ends with
+// w.items == kWalkItems or w.b >= c.bend, or before a node whose test is too
+// close to call by t_yes and t_no or whose span does not advance: the caller
+// takes that step. (Every load is waited for inside; a mask written by a
+// vector compare is read by the scalar unit, or by a vector instruction at
+// least two instructions later.)
+#define PG_WALK_RECORD(WHO, END, MASK)                                                          \
+    "s_mov_b32 m0, %[items]\n\t"                                                                \
+    END                                                                                         \
+    "v_writelane_b32 %[it], " WHO ", m0\n\t"                                                    \
+    "v_mov_b32 %[v0], %[items]\n\t"                                                             \
+    "ds_write_b8 %[entry], %[v0]\n\t"                                                           \
+    "s_add_u32 %[items], %[items], 1\n\t"                                                       \
+    "v_addc_co_u32 %[entry], vcc, 0, %[entry], " MASK "\n\t"
+#define PG_WALK_SKIP_LANES(E)                                                                   \
+    "v_mov_b32 %[v1], " E "\n\t"                                                                \
+    "v_cndmask_b32 %[skip], %[skip], %[v1], %[m]\n\t"
+#define PG_WALK_SET(P, O, REC, CX, CY, CZ, SKIP, LV, SPAN, START, END, OREC, OSPAN, OSTART,     \
+                    NEAR_TEST)                                                                  \
+    "Lw" P "type%=:\n\t"                                                                        \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                                  \
+    "s_cmp_eq_u32 " START ", %[b]\n\t"                                                          \
+    "s_cbranch_scc0 Lw" P "leaf%=\n"                                                            \
+    "Lw" P "node%=:\n\t"                                                                        \
+    "s_lshl_b32 %[st], " SKIP ", 3\n\t"                                                         \
+    "s_load_dwordx8 " OREC ", %[hot], %[st]\n\t"                                                \
+    "s_load_dwordx2 " OSPAN ", %[span], " SKIP "\n\t"                                           \
+    "v_cmp_ge_u32 %[act], %[b], %[skip]\n\t"                                                    \
+    "v_add_f64 %[d0], %[x], -" CX "\n\t"                                                        \
+    "v_add_f64 %[d1], %[y], -" CY "\n\t"                                                        \
+    "v_add_f64 %[d2], %[z], -" CZ "\n\t"                                                        \
+    "v_mul_f64 %[q], %[d0], %[d0]\n\t"                                                          \
+    "v_fma_f64 %[q], %[d1], %[d1], %[q]\n\t"                                                    \
+    "v_fma_f64 %[q], %[d2], %[d2], %[q]\n\t"                                                    \
+    "v_ldexp_f64 %[q], %[q], " LV "\n\t"                                                        \
+    "v_cmp_lt_f64 %[m], %[yes], %[q]\n\t"                                                       \
+    "v_cmp_gt_f64 vcc, %[no], %[q]\n\t"                                                         \
+    "s_or_b64 vcc, vcc, %[m]\n\t"                                                               \
+    "s_andn2_b64 vcc, %[act], vcc\n\t"                                                          \
+    "s_cbranch_scc1 Lwend%=\n\t"                                                                \
+    "s_and_b64 %[m], %[m], %[act]\n\t"                                                          \
+    NEAR_TEST                                                                                   \
+    "s_andn2_b64 vcc, %[act], %[m]\n\t"                                                         \
+    "s_cbranch_scc0 Lw" P "skip%=\n\t"                                                          \
+    /* some lane opened the node */                                                             \
+    "s_cmp_eq_u64 %[m], 0\n\t"                                                                  \
+    "s_cbranch_scc1 Lw" P "none%=\n\t"                                                          \
+    PG_WALK_RECORD("%[k]", PG_WALK_SKIP_LANES(END), "%[m]")                                     \
+    "Lw" P "none%=:\n\t"                                                                        \
+    "s_add_u32 %[k], %[k], 8\n\t"                                                               \
+    "s_lshl_b32 %[st], %[k], 3\n\t"                                                             \
+    "s_load_dwordx8 " REC ", %[hot], %[st]\n\t"                                                 \
+    "s_load_dwordx2 " SPAN ", %[span], %[k]\n\t"                                                \
+    "s_cmp_eq_u32 %[items], 64\n\t"                                                             \
+    "s_cbranch_scc0 Lw" P "type%=\n\t"                                                          \
+    "s_branch Lwend%=\n"                                                                        \
+    /* every lane at the node took it */                                                        \
+    "Lw" P "skip%=:\n\t"                                                                        \
+    "s_cmp_gt_u32 " END ", %[b]\n\t"                                                            \
+    "s_cbranch_scc0 Lwend%=\n\t"                                                                \
+    PG_WALK_RECORD("%[k]", PG_WALK_SKIP_LANES(END), "%[m]")                                     \
+    "s_mov_b32 %[b], " END "\n\t"                                                               \
+    "s_mov_b32 %[k], " SKIP "\n\t"                                                              \
+    "s_cmp_eq_u32 %[items], 64\n\t"                                                             \
+    "s_cbranch_scc1 Lwend%=\n\t"                                                                \
+    "s_cmp_ge_u32 %[b], %[bend]\n\t"                                                            \
+    "s_cbranch_scc1 Lwend%=\n\t"                                                                \
+    "s_waitcnt lgkmcnt(0)\n\t"                                                                  \
+    "s_cmp_eq_u32 " OSTART ", %[b]\n\t"                                                         \
+    "s_cbranch_scc1 Lw" O "node%=\n\t"                                                          \
+    "s_branch Lw" O "leaf%=\n"                                                                  \
+    /* the leaf of body b: at least one lane is at it, as one opened its parent */              \
+    "Lw" P "leaf%=:\n\t"                                                                        \
+    "v_cmp_ge_u32 %[act], %[b], %[skip]\n\t"                                                    \
+    "s_bitset1_b64 %[leaf], %[items]\n\t"                                                       \
+    PG_WALK_RECORD("%[b]", "", "%[act]")                                                        \
+    "s_add_u32 %[b], %[b], 1\n\t"                                                               \
+    "s_cmp_eq_u32 %[items], 64\n\t"                                                             \
+    "s_cbranch_scc1 Lwend%=\n\t"                                                                \
+    "s_cmp_ge_u32 %[b], %[bend]\n\t"                                                            \
+    "s_cbranch_scc1 Lwend%=\n\t"                                                                \
+    "s_cmp_eq_u32 " START ", %[b]\n\t"                                                          \
+    "s_cbranch_scc1 Lw" P "node%=\n\t"                                                          \
+    "s_branch Lw" P "leaf%=\n"
+#define PG_WALK_LOOP(NEAR_A, NEAR_B)                                                            \
+    "s_lshl_b32 %[st], %[k], 3\n\t"                                                             \
+    "s_load_dwordx8 s[64:71], %[hot], %[st]\n\t"                                                \
+    "s_load_dwordx2 s[72:73], %[span], %[k]\n"                                                  \
+    PG_WALK_SET("x", "y", "s[64:71]", "s[64:65]", "s[66:67]", "s[68:69]", "s70", "s71",         \
+                "s[72:73]", "s72", "s73", "s[76:83]", "s[84:85]", "s84", NEAR_A)                \
+    PG_WALK_SET("y", "x", "s[76:83]", "s[76:77]", "s[78:79]", "s[80:81]", "s82", "s83",         \
+                "s[84:85]", "s84", "s85", "s[64:71]", "s[72:73]", "s72", NEAR_B)                \
+    "Lwend%=:\n\t"                                                                              \
+    "s_waitcnt lgkmcnt(0)\n\t"
+// A node within the wave's level bounds: lanes whose own bounds hold its level
+// and that lie within extent 2^-level + margin of its centre on every axis
+// don't take it.
+#define PG_WALK_NEAR(P, LV, Z_TEST)                                                             \
+    "s_cmp_lt_u32 " LV ", %[nlo]\n\t"                                                           \
+    "s_cbranch_scc1 Lw" P "far%=\n\t"                                                           \
+    "s_cmp_gt_u32 " LV ", %[nhi]\n\t"                                                           \
+    "s_cbranch_scc1 Lw" P "far%=\n\t"                                                           \
+    "s_lshr_b32 %[st], " LV ", 1\n\t"                                                           \
+    "s_sub_u32 %[st], 0, %[st]\n\t"                                                             \
+    "v_ldexp_f64 %[q], %[ext], %[st]\n\t"                                                       \
+    "v_add_f64 %[q], %[q], %[mar]\n\t"                                                          \
+    "v_cmp_lt_f64 vcc, |%[d0]|, %[q]\n\t"                                                       \
+    "v_cmp_lt_f64 %[m2], |%[d1]|, %[q]\n\t"                                                     \
+    "s_and_b64 vcc, vcc, %[m2]\n\t"                                                             \
+    Z_TEST                                                                                      \
+    "v_cmp_ge_u32 %[m2], " LV ", %[llo]\n\t"                                                    \
+    "s_and_b64 vcc, vcc, %[m2]\n\t"                                                             \
+    "v_cmp_le_u32 %[m2], " LV ", %[lhi]\n\t"                                                    \
+    "s_and_b64 vcc, vcc, %[m2]\n\t"                                                             \
+    "s_andn2_b64 %[m], %[m], vcc\n"                                                             \
+    "Lw" P "far%=:\n\t"
+#define PG_WALK_Z "v_cmp_lt_f64 %[m2], |%[d2]|, %[q]\n\ts_and_b64 vcc, vcc, %[m2]\n\t"
+template <int DIM, bool NEAR>
+__device__ __forceinline__ void walk_items(WalkState& w, const WalkConst& c) {
+    uint64_t act, m, m2;
+    uint32_t st, v0, v1;
+    double d0, d1, d2, q;
+#define PG_WALK_ASM(CODE, ...)                                                                  \
+    asm volatile(CODE                                                                           \
+                 : [b] "+&s"(w.b), [k] "+&s"(w.k8), [items] "+&s"(w.items), [leaf] "+&s"(w.leaf),   \
+                   [it] "+&v"(w.it), [entry] "+&v"(w.entry), [skip] "+&v"(w.skip_until),           \
+                   [act] "=&s"(act), [m] "=&s"(m), [m2] "=&s"(m2), [st] "=&s"(st),              \
+                   [v0] "=&v"(v0), [v1] "=&v"(v1), [d0] "=&v"(d0), [d1] "=&v"(d1),              \
+                   [d2] "=&v"(d2), [q] "=&v"(q)                                                 \
+                 : [hot] "s"(c.hot), [span] "s"(c.span), [bend] "s"(c.bend),                    \
+                   [yes] "s"(c.t_yes), [no] "s"(c.t_no), [x] "v"(c.x), [y] "v"(c.y),            \
+                   [z] "v"(c.z) __VA_ARGS__                                                     \
+                 : "vcc", "scc", "memory", "s64", "s65", "s66", "s67", "s68", "s69", "s70",     \
+                   "s71", "s72", "s73", "s76", "s77", "s78", "s79", "s80", "s81", "s82",        \
+                   "s83", "s84", "s85")
+#define PG_COMMA ,
+#define PG_NEAR_ARGS                                                                            \
+    PG_COMMA [nlo] "s"(c.near_lo), [nhi] "s"(c.near_hi), [ext] "v"(c.extent),                   \
+        [mar] "v"(c.margin), [llo] "v"(c.lane_lo), [lhi] "v"(c.lane_hi)
+    if constexpr (!NEAR) {
+        PG_WALK_ASM(PG_WALK_LOOP("", ""), );
+    } else if constexpr (DIM == 3) {
+        PG_WALK_ASM(PG_WALK_LOOP(PG_WALK_NEAR("x", "s71", PG_WALK_Z),
+                                 PG_WALK_NEAR("y", "s83", PG_WALK_Z)), PG_NEAR_ARGS);
+    } else {
+        PG_WALK_ASM(PG_WALK_LOOP(PG_WALK_NEAR("x", "s71", ""), PG_WALK_NEAR("y", "s83", "")),
+                    PG_NEAR_ARGS);
+    }
+#undef PG_NEAR_ARGS
+#undef PG_COMMA
+#undef PG_WALK_ASM
+}
+#undef PG_WALK_Z
+#undef PG_WALK_NEAR
+#undef PG_WALK_LOOP
+#undef PG_WALK_SET
+#undef PG_WALK_SKIP_LANES
+#undef PG_WALK_RECORD
 
 template <int DIM, bool FP64, bool INTEGRATE, bool NEAR, bool COUNT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_walk(const SegDesc* __restrict__ desc, uint64_t total,
-                                                 const uint64_t* __restrict__ skeys, int segbits,
-                                                 const uint32_t* __restrict__ first_node,
-                                                 const NodeHot* __restrict__ hot, uint64_t cap,
-                                                 uint32_t nseg, double* __restrict__ acc_out,
-                                                 uint64_t* __restrict__ ext_partial,
-                                                 StepCounters* __restrict__ sc, uint64_t tag,
-                                                 const uint8_t* __restrict__ leaf_lv,
-                                                 uint32_t run_log2,
-                                                 const double4* __restrict__ leafpos,
-                                                 const uint2* __restrict__ node_span,
-                                                 const uint32_t* __restrict__ svals) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) void k_walk(
+    const SegDesc* __restrict__ desc, uint64_t total, const uint64_t* __restrict__ skeys,
+    int segbits, const uint32_t* __restrict__ first_node, const NodeHot* __restrict__ hot,
+    uint64_t cap, uint32_t nseg, double* __restrict__ acc_out, uint64_t* __restrict__ ext_partial,
+    StepCounters* __restrict__ sc, uint64_t tag, const uint8_t* __restrict__ leaf_lv,
+    uint32_t run_log2, const double4* __restrict__ leafpos, const uint2* __restrict__ node_span,
+    const uint32_t* __restrict__ svals) {
+    // per wave: the lanes' lists (item numbers within the chunk) and the
+    // chunk's sources, all (x, y) then all (z, mass): FP32 mass in mixed
+    // precision
+    __shared__ uint32_t s_list[kBlock / 64][64 * kWalkStride];
+    __shared__ double2 s_src[kBlock / 64][2 * kWalkItems];
     // Workgroups go to the 8 XCDs in turn. Each XCD takes runs of 2^run_log2
     // consecutive blocks (16 by default: 4096 sorted bodies), so neighbouring
     // walks share their node records in one L2, while the runs of a batch's
@@ -3109,35 +3285,41 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         blk = (k >> run_log2) * group + (x << run_log2) + (k & ((1u << run_log2) - 1u));
     }
     const uint64_t g = (uint64_t)blk * blockDim.x + threadIdx.x;
-    bool valid = g < total;
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    // Every load that needs no other goes out at once, at indices clamped into
+    // range (a load behind a divergent branch is waited for at the branch's
+    // end); a batch of one segment needs no key to name it, and a wave in one
+    // segment (most are) reads its descriptor through the scalar unit.
+    const uint64_t gc = min(g, total - 1);
+    const uint32_t v = svals[gc];
+    const double4 p = leafpos[gc];
     uint32_t s = 0;
-    double x = 0.0, y = 0.0, z = 0.0, m = 0.0;
-    bool fixed = true;
-    uint64_t j = 0, src = 0;
-    double4 pr = make_double4(0.0, 0.0, 0.0, 0.0);
-    if (valid) {
-        const uint64_t key = skeys[g];
-        const uint32_t v = svals[g];
-        s = seg_of_key(key, segbits);
-        valid = s < nseg;
-        src = v;
-    }
-    if (valid) {
+    if (nseg > 1) s = seg_of_key(skeys[gc], segbits);
+    bool valid = g < total && s < nseg;
+    s = valid ? s : 0u;
+    const uint32_t su = uniform_u32(s);
+    const double4* sprv;
+    uint64_t off, n;
+    if (!lanes_where(s != su)) {
+        const SegDesc& d = desc[su];
+        sprv = d.sprv;
+        off = d.off;
+        n = d.n;
+    } else {
         const SegDesc& d = desc[s];
-        j = g - d.off;
-        // the body's index in the previous order (k_scan_gather flags one
-        // outside its segment; such a body is not stepped)
-        src -= d.off;
-        valid = src < d.n;
+        sprv = d.sprv;
+        off = d.off;
+        n = d.n;
     }
-    if (valid) {
-        const SegDesc& d = desc[s];
-        const double4 p = leafpos[g];
-        x = p.x; y = p.y; z = p.z;
-        m = p.w;
-        pr = gload(d.sprv + src);  // previous position and tag, previous order
-        fixed = tag_fixed(pr.w);
-    }
+    // the body's index in the previous order (k_scan_gather flags one
+    // outside its segment; such a body is not stepped)
+    const uint64_t j = g - off, src = (uint64_t)v - off;
+    valid = valid && src < n;
+    const double4 pr = gload(sprv + (valid ? src : 0));  // previous position and tag
+    const double x = p.x, y = p.y, z = p.z, m = p.w;
+    const bool fixed = !valid || tag_fixed(pr.w);
+    bool history = true;  // the Stormer history holds (a step after the first)
+    uint32_t* list = s_list[wv] + lane * kWalkStride;
     Kahan3 ka;
     ka.zero();
     double f64[3] = {0.0, 0.0, 0.0};
@@ -3148,17 +3330,32 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         const uint32_t s0 = uniform_u32(__shfl(s, lead));
         const bool mine = pending && s == s0;
         const SegDesc& d0 = desc[s0];
-        // the segment's bodies [b, bend) and internal nodes [k, kend) in
+        // the segment's bodies [b, bend) and its first internal node, in
         // preorder (global sorted indices)
         const uint32_t bend = uniform_u32((uint32_t)(d0.off + d0.n));
-        const uint32_t kend = uniform_u32(min((uint64_t)first_node[bend], cap));
-        uint32_t k = uniform_u32(first_node[d0.off]);
-        uint32_t b = uniform_u32((uint32_t)d0.off);
+        const uint32_t k0 = uniform_u32((uint32_t)min((uint64_t)first_node[d0.off], cap));
+        const uint32_t b0 = uniform_u32((uint32_t)d0.off);
         const double E = bits_f64(d0.st->extent_bits);
+        const bool h0 = d0.st->history != 0;
+        history = mine ? h0 : history;
         const double theta = d0.theta;
         const double e = d0.e;
         const float ef = (float)e;
         const bool walker = mine && !fixed;
+        // The opening test `hw / sqrt(s) < theta` (octree.rs:137-140), hw = E
+        // 2^-level, decided exactly: it holds iff s 4^level > (E / theta)^2,
+        // and s formed with fused multiply-adds and the reference's rounded
+        // quotient are within a few 1e-16 of exact, so outside a band of
+        // 1e-10 around the threshold one FP64 comparison decides; inside it
+        // (or where theta or E leave the range in which no step under- or
+        // overflows: thresholds of NaN) the reference's own square root and
+        // division do. 9 vector instructions, where an FP32 quotient with its
+        // band took 25.
+        const double t0 = (E / theta) * (E / theta);
+        const bool plain = theta > 0.0 && E > 0x1p-900 && E < 0x1p+900 && t0 > 0x1p-800 &&
+                           t0 < 0x1p+800;
+        const double t_yes = scalar_f64(plain ? t0 * (1.0 + 1e-10) : __builtin_nan(""));
+        const double t_no = scalar_f64(plain ? t0 * (1.0 - 1e-10) : __builtin_nan(""));
         // near field (no reference counterpart; off at 0): a cell at the
         // scale of the body's own leaf cell (its level and the kNearLevels
         // below) is opened, never taken whole, when the body lies within
@@ -3170,76 +3367,120 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         // (NEAR: some segment of the batch has one; the walk without the
         // test holds fewer registers)
         const bool nearf = NEAR && d0.near > 0.0;
-        const int lleaf = nearf && walker ? (int)leaf_lv[g] : 0;
-        const double margin = nearf && walker ? d0.near * ldexp(E, 1 - lleaf) : 0.0;
-        uint32_t skip_until = 0;  // a lane skips the items of the bodies below this
+        const uint32_t lleaf = nearf && walker ? (uint32_t)leaf_lv[g] : 0u;
+        const double margin = nearf && walker ? d0.near * ldexp(E, 1 - (int)lleaf) : 0.0;
+        WalkConst wc{hot, node_span, bend, t_yes, t_no, x, y, z, ~0u, 0u, E, margin,
+                     2u * lleaf, 2u * (lleaf + kNearLevels)};
+        if (nearf) {
+            // the levels at which some lane's near field opens cells
+            wc.near_lo = 2u * uniform_u32(__shfl(
+                                  wave_incl_scan_u32(walker ? lleaf : 255u, 255u, OpMin{}), 63));
+            wc.near_hi = 2u * (kNearLevels + 255u -
+                               uniform_u32(__shfl(wave_incl_scan_u32(walker ? 255u - lleaf : 255u,
+                                                                     255u, OpMin{}), 63)));
+        }
         // The walk visits the tree in preorder as two merged sequences: the
         // next item is internal node k when k starts at body b (its span's
         // first body), else the leaf of body b. After node k the next item is
         // (b, k + 1) when some lane opened it, else (the body after its
-        // range, its skip). The next record is loaded once the lanes have
-        // decided (index clamped into the node array; a record past kend is
-        // never used). Each step raises b or k (guarded against a corrupt
-        // record), so the loop ends.
-        const uint32_t clamp = (uint32_t)(cap - 1);
-        NodeHot h = at32(hot, min(k, clamp));
-        uint2 sp = at32(node_span, min(k, clamp));
-        while (b < bend) {
-            // this item's source (a taken node's centre of mass and mass, or
-            // a leaf's body) and whether this lane adds it
-            double bx, by, bz, bm;
-            bool add = false;
-            if (k < kend && sp.x == b) {
-                bx = vcopy(h.mx); by = vcopy(h.my); bz = vcopy(h.mz); bm = vcopy(h.mass);
-                // the opening test for every lane, its result kept by the
-                // lanes still walking (no branch on the common path)
-                const bool act = walker && b >= skip_until;
-                const double d0x = x - h.cx, d0y = y - h.cy, d0z = z - h.cz;
-                // (the level is taken from the record where it is used: left
-                // to itself the compiler extracts it right after the next
-                // record's load, which makes that load wait at once)
-                int lvw;
-                asm("s_and_b32 %0, %1, 0xffff" : "=s"(lvw) : "s"(h.lvl_oct) : "scc");
-                const double hw = ldexp(E, -lvw);
-                bool take = accept_cell(hw, d0x * d0x + d0y * d0y + d0z * d0z, theta, act);
+        // range, its skip). k is at most the last internal node of the batch
+        // plus one, whose span (k_tree_scan) starts at no body. Each step
+        // raises b, or k at the same b, so the walk ends.
+        WalkState w;
+        w.b = lanes_where(walker) ? b0 : bend;
+        w.k8 = 8u * k0;
+        // a lane skips the items of the bodies below this (all, if it does
+        // not walk)
+        w.skip_until = walker ? 0u : ~0u;
+        while (w.b < bend) {
+            // (1) up to kWalkItems items; a lane writes each item's number at
+            // its list's end and keeps it there if it takes the item
+            const uint32_t entry0 = lds_address(list);
+            w.items = 0;
+            w.leaf = 0;
+            w.it = 0;
+            w.entry = entry0;
+            for (;;) {
+                walk_items<DIM, NEAR>(w, wc);
+                if (w.items == kWalkItems || w.b >= bend) break;
+                // a node whose test the thresholds do not decide: the step
+                // with the reference's own square root and division
+                const uint32_t k = w.k8 >> 3;
+                const NodeHot& h = at32(hot, k);
+                const uint2 sp = at32(node_span, k);
+                const uint32_t lv = uniform_u32(h.level2) >> 1;
+                const double dx = x - h.cx, dy = y - h.cy, dz = z - h.cz;
+                const double hw = ldexp(E, -(int)lv);
+                const uint64_t act = lanes_where(w.b >= w.skip_until);
+                uint64_t take =
+                    act & lanes_where(hw / sqrt(dx * dx + dy * dy + dz * dz) < theta);
                 if (nearf) {
-                    const int lv = lvw;
                     const double reach = hw + margin;
-                    const bool close = fabs(d0x) < reach && fabs(d0y) < reach &&
-                                       (DIM == 2 || fabs(d0z) < reach);
-                    take = take && !(lv >= lleaf && lv <= lleaf + kNearLevels && close);
+                    const bool close = fabs(dx) < reach && fabs(dy) < reach &&
+                                       (DIM == 2 || fabs(dz) < reach);
+                    take &= ~lanes_where(lv >= lleaf && lv <= lleaf + kNearLevels && close);
                 }
-                take = take && act;
-                const bool open = act && !take;
-                skip_until = take ? sp.y : skip_until;
-                add = take;
-                // the next item's index by selects (one pair of record loads,
-                // no branch: each branch cost scalar instructions)
-                const bool go_open = __ballot(open) || h.skip <= k || sp.y <= b;
-                const uint32_t kn = go_open ? k + 1u : h.skip;
-                b = uniform_u32(go_open ? b : sp.y);
-                k = uniform_u32(kn);
-                h = at32(hot, min(k, clamp));
-                sp = at32(node_span, min(k, clamp));
-            } else {
-                // the leaf of body b: its exact position and mass
-                const double4 lp = at32(leafpos, b);
-                bx = lp.x; by = lp.y; bz = lp.z; bm = lp.w;
-                add = walker && b >= skip_until;
-                b = uniform_u32(b + 1u);
-            }
-            // (the reference skips a source at the body's own position)
-            const bool other = !(bx == x && by == y && bz == z);
-            if (FP64) {
-                if (add) {
-                    if (COUNT) ++count;
-                    if (other) pair_fp64(x, y, z, m, bx, by, bz, bm, e, f64);
+                if (take) {
+                    w.skip_until = lane_in(take) ? sp.y : w.skip_until;
+                    w.it = write_lane(w.it, w.k8, w.items);
+                    reinterpret_cast<uint8_t*>(list)[w.entry - entry0] = (uint8_t)w.items;
+                    w.entry += lane_in(take) ? 1u : 0u;
+                    w.items = uniform_u32(w.items + 1u);
                 }
-            } else {
-                // (every lane forms the term; the lanes that add keep it)
-                if (COUNT) count += add ? 1u : 0u;
-                pair_mixed(x, y, z, bx, by, bz, bm, ef, ka, add, other);
+                const bool opened = (act & ~take) != 0;
+                w.k8 = uniform_u32(opened ? w.k8 + 8u : h.skip8);
+                w.b = uniform_u32(opened ? w.b : max(sp.y, w.b + 1u));
+                if (w.items == kWalkItems || w.b >= bend) break;
             }
+            // (2) the items' sources, one per lane, then each lane's own list
+            // in order
+            const uint32_t cnt = w.entry - entry0;
+            if (COUNT) count += cnt;
+            if (lane < w.items) {
+                const double4 q = gload((w.leaf >> lane) & 1ull
+                                            ? leafpos + w.it
+                                            : reinterpret_cast<const double4*>(&hot[w.it >> 3].mx));
+                s_src[wv][lane] = make_double2(q.x, q.y);
+                s_src[wv][kWalkItems + lane] =
+                    make_double2(q.z, FP64 ? q.w : bits_f64((uint64_t)f32_bits((float)q.w)));
+            }
+            wave_lds_sync();
+            for (uint32_t t = 0; lanes_where(t < cnt); t += 4u) {
+                const uint32_t q = list[t >> 2];
+                if (FP64) {
+#pragma unroll 1
+                    for (uint32_t u = 0; u < 4u; ++u) {
+                        // (an entry past a lane's count may hold anything:
+                        // any six bits name a source, whose term is dropped)
+                        const uint32_t i = (q >> (8u * u)) & (kWalkItems - 1u);
+                        const double2 a = s_src[wv][i], c = s_src[wv][kWalkItems + i];
+                        // (the reference skips a source at the body's own
+                        // position)
+                        if (t + u < cnt && !(a.x == x && a.y == y && c.x == z))
+                            pair_fp64(x, y, z, m, a.x, a.y, c.x, c.y, e, f64);
+                    }
+                } else {
+                    float3 v[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; ++u) {
+                        // (an entry past a lane's count may hold anything:
+                        // any six bits name a source, whose term is dropped)
+                        const uint32_t i = (q >> (8u * u)) & (kWalkItems - 1u);
+                        const double2 a = s_src[wv][i], c = s_src[wv][kWalkItems + i];
+                        v[u] = pair_mixed(x, y, z, a.x, a.y, c.x,
+                                          bits_f32((uint32_t)f64_bits(c.y)), ef);
+                    }
+                    // (four terms formed together, and not each where a lane
+                    // that has the entry adds it)
+                    asm volatile("" : "+v"(v[0].x), "+v"(v[0].y), "+v"(v[0].z), "+v"(v[1].x),
+                                 "+v"(v[1].y), "+v"(v[1].z), "+v"(v[2].x), "+v"(v[2].y),
+                                 "+v"(v[2].z), "+v"(v[3].x), "+v"(v[3].y), "+v"(v[3].z));
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; ++u)
+                        if (t + u < cnt) ka.add(v[u].x, v[u].y, v[u].z);
+                }
+            }
+            wave_lds_sync();
         }
         pending = pending && !mine;
     }
@@ -3281,7 +3522,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
             const double dt = d.dt;
             const double dt2 = dt * dt;
             double nx, ny, nz;
-            if (d.st->history == 0) {
+            if (!history) {
                 const double ux = gload(d.dvx + j), uy = gload(d.dvy + j), uz = gload(d.dvz + j);
                 nx = x + ux * dt + 0.5 * ax * dt2;
                 ny = y + uy * dt + 0.5 * ay * dt2;
