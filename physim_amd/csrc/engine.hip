@@ -152,7 +152,7 @@ struct pg_engine {
     // per-call host tables of run_batch, kept so that a call whose sizes fit
     // what earlier calls held allocates nothing on the host either
     std::vector<pg_sim*> h_sims;
-    std::vector<uint32_t> h_nsplit, h_chunk0, h_nchunk, h_tile0;
+    std::vector<uint32_t> h_chunk0, h_nchunk, h_tile0;
     std::vector<uint64_t> h_part_off;
 };
 
@@ -607,17 +607,43 @@ static void ev_collect(pg_engine* e) {
 }
 
 // ---------------------------------------------------------- step sequence
-// Source splits of a direct-sum segment of n bodies: small segments are too
-// few target tiles to fill the GPU, so up to kMaxDirectSplit blocks share a
-// target tile, each summing a contiguous range of source tiles. The count
-// follows from the segment's own size, so a segment sums alike alone and in
-// a batch.
+// How the blocks of a direct-sum segment of n bodies share a target tile's
+// sources: small segments are too few target tiles to fill the GPU, so up to
+// 2^19 / n blocks share one, each summing a group of sources (2,048 blocks in
+// all, eight waves a SIMD; where at most four shared one, 1,000, 8,195 and
+// 32,770 bodies took 94, 700 and 6,910 us in FP64, 20, 199 and 2,690 now with
+// their shared divisions, and 22, 116 and 873 us in mixed precision, 21, 60 and
+// 862 now). The partial sums take
+// at most kDirectPartBytes, what the allocation-free transform's node array
+// holds. In mixed precision the compensated sums run over kMaxDirectSplit
+// ranges of tiles whatever the groups, so that every size keeps the sums it had
+// with one block per range; more groups than ranges write each tile's partial
+// sum, which fits up to 18,900 bodies. All follow from the segment's own size,
+// so a segment sums alike alone and in a batch.
 constexpr uint32_t kMaxDirectSplit = 4;
-static uint32_t direct_splits(uint64_t n) {
-    const uint64_t tiles = (n + kBlock - 1) / kBlock;
-    uint64_t s = n ? ((1ull << 19) + n - 1) / n : 1;
-    s = std::min<uint64_t>(std::min<uint64_t>(s, kMaxDirectSplit), tiles);
-    return (uint32_t)std::max<uint64_t>(s, 1);
+constexpr uint64_t kDirectPartBytes = 16ull << 20;
+struct DirectSplit {
+    uint32_t ranges = 1, groups = 1;
+    bool fine = false;
+    uint64_t parts = 0;  // partial sums (24 bytes each)
+};
+static DirectSplit direct_split(uint64_t n, bool fp64) {
+    DirectSplit d;
+    const uint64_t tiles = std::max<uint64_t>((n + kBlock - 1) / kBlock, 1);
+    const uint64_t fill = n ? ((1ull << 19) + n - 1) / n : 1;  // blocks per target tile
+    d.ranges = (uint32_t)std::min<uint64_t>(std::min(fill, tiles), kMaxDirectSplit);
+    d.groups = d.ranges;
+    if (fp64) {
+        const uint64_t units = (n + kDirectUnit - 1) / kDirectUnit;
+        const uint64_t hold = kDirectPartBytes / (24 * std::max<uint64_t>(n, 1));
+        d.groups = (uint32_t)std::max<uint64_t>(
+            d.ranges, std::min<uint64_t>({fill, units, hold, 255}));
+    } else if (std::min(fill, tiles) > d.ranges && tiles * n * 12 <= kDirectPartBytes) {
+        d.groups = (uint32_t)std::min<uint64_t>({fill, tiles, 255});
+        d.fine = true;
+    }
+    if (d.groups > 1) d.parts = d.fine ? (tiles * n + 1) / 2 : d.groups * n;
+    return d;
 }
 
 struct BatchPlan {
@@ -631,7 +657,7 @@ struct BatchPlan {
     uint32_t nblocks = 0;
     uint32_t nchunks = 0;
     uint32_t ntiles = 0;  // node tiles
-    uint32_t max_split = 1;  // direct sum: the most source splits of a segment
+    uint32_t max_group = 1;  // direct sum: the most source groups of a segment
     bool integrate = true;
     bool near = false;   // some segment walks with a near field (the walk that tests for it)
     bool count = false;  // some segment counts interactions (the walk that counts)
@@ -809,7 +835,7 @@ static void enqueue_direct_step(pg_engine* e, const BatchPlan& bp, int q, bool c
         double* part = reinterpret_cast<double*>(e->hot);
         k_direct<FP64, INTEG><<<bp.nblocks, kBlock, 0, st>>>(desc, e->blk_seg, e->blk_tile,
                                                             part, e->acc_out);
-        if (bp.max_split > 1)
+        if (bp.max_group > 1)
             k_direct_finish<FP64, INTEG><<<grid_for(bp.total, 1u << 30), kBlock, 0, st>>>(
                 desc, e->seg_off, bp.nseg, bp.total, part, e->acc_out);
     });
@@ -921,30 +947,24 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     if (nodes >= (1ull << 32)) return pg_set_error(PG_ERR_ARG, "tree too large for 32-bit nodes");
     e->h_blk_seg.clear();
     e->h_blk_tile.clear();
-    std::vector<uint32_t>& nsplit = e->h_nsplit;
     std::vector<uint64_t>& part_off = e->h_part_off;
-    nsplit.assign(bp.nseg, 1u);
     part_off.assign(bp.nseg, 0ull);
     if (bp.kind == PG_KIND_DIRECT) {
-        // Blocks: per segment, target tile and source split (split in the
-        // tile word's top 8 bits). A segment's partial sums (3 doubles per
-        // body and split) live in the node array, which the direct sum does
-        // not otherwise use.
+        // Blocks: per segment, target tile and source group (group in the
+        // tile word's top 8 bits). A segment's partial sums live in the node
+        // array, which the direct sum does not otherwise use.
         uint64_t part = 0;
         for (uint32_t s = 0; s < bp.nseg; ++s) {
             const uint32_t nb = (uint32_t)((sims[s]->n + kBlock - 1) / kBlock);
-            const uint32_t S = direct_splits(sims[s]->n);
+            const DirectSplit ds = direct_split(sims[s]->n, bp.precision == PG_PREC_FP64);
             for (uint32_t t = 0; t < nb; ++t)
-                for (uint32_t p = 0; p < S; ++p) {
+                for (uint32_t p = 0; p < ds.groups; ++p) {
                     e->h_blk_seg.push_back(s);
                     e->h_blk_tile.push_back(t | (p << 24));
                 }
-            nsplit[s] = S;
-            if (S > 1) {
-                part_off[s] = part;
-                part += (uint64_t)S * sims[s]->n;
-                bp.max_split = std::max(bp.max_split, S);
-            }
+            part_off[s] = part;
+            part += ds.parts;
+            bp.max_group = std::max(bp.max_group, ds.groups);
         }
         bp.nblocks = (uint32_t)e->h_blk_seg.size();
         nodes = (part * 24 + sizeof(NodeHot) - 1) / sizeof(NodeHot);
@@ -998,6 +1018,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     uint64_t off = 0;
     for (uint32_t s = 0; s < bp.nseg; ++s) {
         pg_sim* sm = sims[s];
+        const DirectSplit ds = direct_split(sm->n, bp.precision == PG_PREC_FP64);
         e->h_seg_off[s] = off;
         for (int q = 0; q < 2; ++q) {
             const int src = sm->cur ^ q;
@@ -1019,7 +1040,9 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
             d.chunk0 = chunk0[s];
             d.nchunks = nchunk[s];
             d.tile0 = tile0[s];
-            d.nsplit = nsplit[s];
+            d.nsplit = ds.ranges;
+            d.ngroup = ds.groups;
+            d.fine = ds.fine ? 1u : 0u;
             d.part_off = part_off[s];
             d.near = sm->near;
         }
@@ -1627,7 +1650,12 @@ extern "C" int pg_sim_energy(pg_sim* s, double out[6]) {
     const uint64_t n = s->n;
     for (int i = 0; i < 6; ++i) out[i] = 0.0;
     if (!n) return PG_OK;
-    const unsigned nb = (unsigned)((n + kBlock - 1) / kBlock);
+    // block rows times source groups: 2,048 blocks (eight waves a SIMD) where
+    // there are that many groups of kDirectUnit sources to share
+    const unsigned rows = (unsigned)((n + kBlock - 1) / kBlock);
+    const unsigned groups = std::min((unsigned)((n + kDirectUnit - 1) / kDirectUnit),
+                                     (2048u + rows - 1) / rows);
+    const unsigned nb = rows * groups;
     double* part = nullptr;
     HIP_TRY(hipMalloc(&part, (size_t)nb * 5 * 8));
     const int c = s->cur;
@@ -1637,7 +1665,7 @@ extern "C" int pg_sim_energy(pg_sim* s, double out[6]) {
         (void)hipFree(part);
         return vrc;
     }
-    k_energy<<<nb, kBlock, 0, e->stream>>>(s->pos[c], vs, n, std::fabs(s->p.e), part);
+    k_energy<<<dim3(rows, groups), kBlock, 0, e->stream>>>(s->pos[c], vs, n, std::fabs(s->p.e), part);
     hipError_t le = hipGetLastError();
     std::vector<double> h((size_t)nb * 5);
     hipError_t ce = hipMemcpyAsync(h.data(), part, h.size() * 8, hipMemcpyDeviceToHost, e->stream);
@@ -1849,7 +1877,11 @@ static int noalloc_setup(NoAllocCtx& c, int device, hipStream_t stream) {
     const uint64_t state_sz = align256(state_bytes(n));
     const uint64_t stage_sz = align256(n * 24);
     const uint64_t nodes = n * kNoAllocNodesPerBody;
-    const uint32_t blocks = (uint32_t)((n + kBlock - 1) / kBlock) * kMaxDirectSplit;
+    // (ceil(n / 256) target tiles times at most 2^19 / n + 1 blocks, 255 of a
+    // tile's and no more than it has groups of kDirectUnit sources)
+    const uint32_t blocks = (1u << 19) / kBlock + 4 * (uint32_t)((n + kBlock - 1) / kBlock);
+    static_assert(kNoAllocMaxBodies * kNoAllocNodesPerBody * sizeof(NodeHot) >= kDirectPartBytes,
+                  "the direct sum's partial sums in the node array");
     pg_engine& e = c.eng;
     const uint64_t need = state_sz + stage_sz + carve_scratch(&e, nullptr, n, nodes, 1, blocks);
     if (need > kNoAllocBytes)
@@ -1868,7 +1900,6 @@ static int noalloc_setup(NoAllocCtx& c, int device, hipStream_t stream) {
     PG_TRY(clear_scratch_status(&e));
     const uint64_t chunks = n / kExtentChunk + 2, tiles = n / kNodeTile + 2;
     e.h_sims.reserve(1);
-    e.h_nsplit.reserve(1);
     e.h_part_off.reserve(1);
     e.h_chunk0.reserve(1);
     e.h_nchunk.reserve(1);

@@ -39,6 +39,7 @@ constexpr int kTopSlots = 65;      // tree levels 0..64: one tile-spanning node 
 constexpr int kMaxTieRun = 256;    // longest run of equal keys ordered by their deep keys
 constexpr int kMaxLcp = 64;        // deepest common prefix, in levels, of two bodies: the
                                    // reference recurses to depth 64 (octree.rs:60-62)
+constexpr int kDirectUnit = 32;    // sources per group of the FP64 direct sum: a multiple of this
 constexpr int kDeepWords = 3;      // words of a tied body's deep key
 static_assert(kMaxLcp + 1 == kTopSlots, "every level of an internal node has its slot");
 
@@ -96,8 +97,10 @@ struct SegDesc {
     uint32_t chunk0;  // first extent chunk of this segment
     uint32_t nchunks;
     uint32_t tile0;   // first node tile of this segment (node tiles start at its first body)
-    uint32_t nsplit;  // direct sum: blocks summing one target tile, each over a range of sources
-    uint64_t part_off;  // direct sum with nsplit > 1: first partial sum (x3 doubles) of the segment
+    uint32_t nsplit;  // direct sum, mixed precision: ranges of source tiles summed apart
+    uint32_t ngroup;  // direct sum: blocks summing one target tile, each over a group of source tiles
+    uint32_t fine;    // mixed precision: more groups than ranges (every tile's partial sum is kept)
+    uint64_t part_off;  // direct sum with ngroup > 1: first partial sum (x3 doubles) of the segment
     double near;      // near field in widths of the body's own leaf cell (0: off)
 };
 

@@ -3686,12 +3686,14 @@ __device__ __forceinline__ void direct_store(const SegDesc& d, uint64_t i, doubl
 }
 
 // simple_astro (transformers.rs:219-244): LDS-tiled all-pairs sum. Each block
-// holds 256 targets of one segment and streams a range of the segment's
-// sources through LDS: all of them, or one of d.nsplit contiguous ranges of
-// source tiles (the tile word's top 8 bits), whose partial sums k_direct_finish
-// adds in range order. Mixed precision sums each 256-source tile in FP32 and
-// adds the tile partial into a compensated FP32 sum. Reads src, writes dst
-// (same order).
+// holds 256 targets of one segment and streams a group of the segment's
+// sources through LDS: all of them, or one of d.ngroup contiguous groups (the
+// tile word's top 8 bits) of whole source tiles (FP64: of kDirectUnit
+// sources), whose partial sums k_direct_finish adds in order. Mixed precision sums each 256-source tile in FP32 and adds the tile
+// partial into a compensated FP32 sum over one of d.nsplit ranges of tiles;
+// with more groups than ranges (d.fine) each tile's partial is written out and
+// k_direct_finish forms the same compensated sums. Reads src, writes dst (same
+// order).
 template <bool FP64, bool INTEGRATE>
 __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ desc,
                                                    const uint32_t* __restrict__ blk_seg,
@@ -3703,10 +3705,12 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
     const SegDesc& d = desc[s];
     const uint32_t tw = blk_tile[blockIdx.x];
     const uint64_t i = (uint64_t)(tw & 0xFFFFFFu) * kBlock + threadIdx.x;
-    const uint32_t sp = tw >> 24, ns = d.nsplit;
-    const uint64_t src_tiles = (d.n + kBlock - 1) / kBlock;
-    const uint64_t j0 = src_tiles * sp / ns * kBlock;
-    const uint64_t j1 = min(src_tiles * (sp + 1) / ns * kBlock, d.n);
+    const uint32_t sp = tw >> 24, ng = d.ngroup;
+    const bool fine = !FP64 && d.fine != 0;
+    constexpr uint64_t kUnit = FP64 ? kDirectUnit : kBlock;
+    const uint64_t units = (d.n + kUnit - 1) / kUnit;
+    const uint64_t j0 = units * sp / ng * kUnit;
+    const uint64_t j1 = min(units * (sp + 1) / ng * kUnit, d.n);
     const bool valid = i < d.n;
     double x = 0.0, y = 0.0, z = 0.0, m = 0.0;
     bool fixed = true;
@@ -3732,6 +3736,7 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
         __syncthreads();
         const int cnt = (int)min((uint64_t)kBlock, j1 - t0);
         if (FP64) {
+#pragma unroll 4
             for (int k = 0; k < cnt; ++k) {
                 const double4 b = sj[k];
                 pair_fp64(x, y, z, m, b.x, b.y, b.z, b.w, e, f64);
@@ -3756,11 +3761,19 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
                 py = fmaf(fy, w, py);
                 pz = fmaf(fz, w, pz);
             }
-            ka.add(px, py, pz);
+            if (fine) {
+                if (valid) {
+                    float* o = reinterpret_cast<float*>(part + 3 * d.part_off) +
+                               3 * (t0 / kBlock * d.n + i);
+                    o[0] = px; o[1] = py; o[2] = pz;
+                }
+            } else {
+                ka.add(px, py, pz);
+            }
         }
         __syncthreads();
     }
-    if (!valid) return;
+    if (!valid || fine) return;
     double fx, fy, fz;
     if (FP64) {
         fx = f64[0]; fy = f64[1]; fz = f64[2];
@@ -3769,7 +3782,7 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
         fy = (double)ka.sy - (double)ka.cy;
         fz = (double)ka.sz - (double)ka.cz;
     }
-    if (ns > 1) {
+    if (ng > 1) {
         double* o = part + 3 * (d.part_off + (uint64_t)sp * d.n + i);
         o[0] = fx; o[1] = fy; o[2] = fz;
         return;
@@ -3778,7 +3791,8 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
 }
 
 // Bodies of segments whose sources k_direct split: the partial sums added in
-// range order, then the store.
+// group order (or, d.fine, the tiles' compensated sums of each range, added in
+// range order), then the store.
 template <bool FP64, bool INTEGRATE>
 __global__ __launch_bounds__(kBlock) void k_direct_finish(const SegDesc* __restrict__ desc,
                                                           const uint64_t* __restrict__ seg_off,
@@ -3788,13 +3802,32 @@ __global__ __launch_bounds__(kBlock) void k_direct_finish(const SegDesc* __restr
     const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= total) return;
     const SegDesc& d = desc[seg_of(seg_off, nseg, g)];
-    const uint32_t ns = d.nsplit;
-    if (ns <= 1) return;
+    const uint32_t ng = d.ngroup;
+    if (ng <= 1) return;
     const uint64_t i = g - d.off;
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    for (uint32_t sp = 0; sp < ns; ++sp) {
-        const double* o = part + 3 * (d.part_off + (uint64_t)sp * d.n + i);
-        fx += o[0]; fy += o[1]; fz += o[2];
+    if (!FP64 && d.fine) {
+        const uint64_t tiles = (d.n + kBlock - 1) / kBlock;
+        const float* o = reinterpret_cast<const float*>(part + 3 * d.part_off) + 3 * i;
+        for (uint32_t sp = 0; sp < d.nsplit; ++sp) {
+            Kahan3 ka;
+            ka.zero();
+            const uint64_t t1 = tiles * (sp + 1) / d.nsplit;
+#pragma unroll 4
+            for (uint64_t t = tiles * sp / d.nsplit; t < t1; ++t) {
+                const float* v = o + 3 * t * d.n;
+                ka.add(v[0], v[1], v[2]);
+            }
+            fx += (double)ka.sx - (double)ka.cx;
+            fy += (double)ka.sy - (double)ka.cy;
+            fz += (double)ka.sz - (double)ka.cz;
+        }
+    } else {
+#pragma unroll 4
+        for (uint32_t sp = 0; sp < ng; ++sp) {
+            const double* o = part + 3 * (d.part_off + (uint64_t)sp * d.n + i);
+            fx += o[0]; fy += o[1]; fz += o[2];
+        }
     }
     const double4 p = d.spos[i];
     direct_store<FP64, INTEGRATE>(d, i, p.x, p.y, p.z, p.w, tag_fixed(d.sprv[i].w), fx, fy, fz,
@@ -3825,7 +3858,13 @@ struct VelocitySource {
 
 // FP64 energy terms of one state: per block partial sums of
 // {V (half of the all-pairs sum), K, Px, Py, Pz}. U(r) = -(ma mb / sqrt(e))
-// atan(sqrt(e) / r) is the potential of |F| = ma mb / (r^2 + e).
+// atan(sqrt(e) / r) is the potential of |F| = ma mb / (r^2 + e). A block row
+// (blockIdx.x) holds 256 bodies; each of its gridDim.y blocks sums one group of
+// sources, and the first one the kinetic terms. (Vector issue of the square
+// root, division and arctangent bounds it once the chip is full; with one block
+// per row, 1,000, 8,195 and 65,539 bodies ran on 4, 33 and 256 CUs, a wave a
+// SIMD: calls of 380, 2,780 and 35,500 us -> 64, 389
+// and 17,600.)
 __global__ __launch_bounds__(kBlock) void k_energy(const double4* __restrict__ pos,
                                                    VelocitySource vs, uint64_t n,
                                                    double e, double* __restrict__ partial) {
@@ -3840,11 +3879,14 @@ __global__ __launch_bounds__(kBlock) void k_energy(const double4* __restrict__ p
     }
     const double se = sqrt(e);
     double V = 0.0;
-    for (uint64_t t0 = 0; t0 < n; t0 += kBlock) {
+    const uint64_t units = (n + kDirectUnit - 1) / kDirectUnit;
+    const uint64_t j0 = units * blockIdx.y / gridDim.y * kDirectUnit;
+    const uint64_t j1 = min(units * (blockIdx.y + 1) / gridDim.y * kDirectUnit, n);
+    for (uint64_t t0 = j0; t0 < j1; t0 += kBlock) {
         const uint64_t jj = t0 + threadIdx.x;
-        if (jj < n) sj[threadIdx.x] = pos[jj];
+        if (jj < j1) sj[threadIdx.x] = pos[jj];
         __syncthreads();
-        const int cnt = (int)min((uint64_t)kBlock, n - t0);
+        const int cnt = (int)min((uint64_t)kBlock, j1 - t0);
         if (valid) {
             for (int k = 0; k < cnt; ++k) {
                 const double4 b = sj[k];
@@ -3858,7 +3900,7 @@ __global__ __launch_bounds__(kBlock) void k_energy(const double4* __restrict__ p
         __syncthreads();
     }
     double K = 0, Px = 0, Py = 0, Pz = 0;
-    if (valid) {
+    if (valid && blockIdx.y == 0) {
         double vx, vy, vz;
         vs.at(i, xi, yi, zi, vx, vy, vz);
         K = 0.5 * mi * (vx * vx + vy * vy + vz * vz);
@@ -3875,7 +3917,8 @@ __global__ __launch_bounds__(kBlock) void k_energy(const double4* __restrict__ p
             for (int c = 0; c < 5; ++c) red[c][threadIdx.x] += red[c][threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x < 5) partial[5 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
+    if (threadIdx.x < 5)
+        partial[5 * (blockIdx.y * gridDim.x + blockIdx.x) + threadIdx.x] = red[threadIdx.x][0];
 }
 
 // AoS <-> SoA at the host boundary.

@@ -47,3 +47,49 @@ def test_one_term_bit_exact(engine, scale, mass, e):
         a = sim.accel()
         np.testing.assert_array_equal(a, O.simple_transform(s, e))
         sim.close()
+
+
+@pytest.mark.parametrize("n", [256, 257, 1024, 1025, 1537, 4097, 8195, 18900, 19200])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_source_groups(engine, n, precision):
+    rng = np.random.default_rng(n)
+    s = bodies(rng.uniform(-1.0, 1.0, (n, 3)), rng.uniform(0.5, 1.5, n) / n)
+    sim = P.Sim(engine, s, kind="simple_astro", precision=precision, e=0.1)
+    a = sim.accel()
+    rows = np.unique(np.concatenate([np.arange(0, n, max(1, n // 97)), [n - 1]]))
+    ref = O.simple_transform_rows(s, 0.1, rows)
+    pos = np.stack([s["x"], s["y"], s["z"]], 1)
+    r2 = ((pos[rows, None] - pos[None]) ** 2).sum(-1)
+    size = (s["mass"] / (r2 + 0.1)).sum(1)  # the sum of the terms' magnitudes
+    bound = (n * 2.0 ** -53 if precision == "fp64" else 1e-6) * size
+    assert (np.abs(a[rows] - ref).max(1) <= bound).all()
+    # alone, in a batch and through the allocation-free call: the same bits
+    small = bodies(rng.uniform(-1.0, 1.0, (300, 3)), np.full(300, 1.0 / 300))
+    kw = dict(kind="simple_astro", precision=precision, e=0.1, dt=1e-4)
+    pair = [P.Sim(engine, x, **kw) for x in (small, s)]
+    engine.batch_step(pair, 2)
+    one = P.Sim(engine, s, **kw)
+    one.step(2)
+    np.testing.assert_array_equal(pair[1].download(), one.download())
+    b = engine.transform_noalloc(s, kind="simple_astro", e=0.1, precision=precision)
+    np.testing.assert_array_equal(b.view(np.float64).reshape(n, 3), a)
+    for x in pair + [one, sim]:
+        x.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 700])
+def test_energy_groups(engine, n):
+    """Energy terms summed in groups against the oracle's: (n + 1000) 2^-53
+    of the sum of their magnitudes."""
+    rng = np.random.default_rng(n)
+    s = bodies(rng.uniform(-1.0, 1.0, (n, 3)), rng.uniform(0.5, 1.5, n) / n)
+    for f in ("vx", "vy", "vz"):
+        s[f] = rng.normal(size=n)
+    sim = P.Sim(engine, s, kind="simple_astro", e=0.1)
+    got = sim.energy()
+    ref = np.asarray(O.energy(s, 0.1))
+    speed = np.sqrt(s["vx"] ** 2 + s["vy"] ** 2 + s["vz"] ** 2)
+    size = np.array([abs(ref[0]), abs(ref[1]), abs(ref[0]) + abs(ref[1])] +
+                    [float((s["mass"] * speed).sum())] * 3)
+    assert (np.abs(got - ref[:6]) <= (n + 1000) * 2.0 ** -53 * size).all()
+    sim.close()
