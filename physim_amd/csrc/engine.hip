@@ -2,6 +2,7 @@
 // per-kernel event timing and host-boundary conversions. Kernels live in
 // pg_kernels.h.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <chrono>
@@ -146,6 +147,21 @@ struct pg_engine {
     // transient simulation of the transform path
     pg_sim* xform = nullptr;
 
+    // pinned host memory: a call's tables on their way to the device and its
+    // status on the way back (grown with the batch, freed with the engine),
+    // and two halves through which states go up and results come back
+    char* pin = nullptr;
+    uint64_t pin_bytes = 0;
+    char* ret = nullptr;
+    uint64_t ret_half = 0;
+    hipEvent_t ret_ev[2] = {nullptr, nullptr};
+    // the descriptors the device tables were last written from (both
+    // parities) and their kind; none when empty
+    std::vector<SegDesc> up_desc[2];
+    int up_kind = -1, up_prec = -1;
+    bool pin_busy = false;  // tables in pinned memory may still be read by the stream
+    uint64_t pending = 0;  // segments whose status the next finish_batch reads
+
     // the scratch is the library's static device array (allocation-free
     // transform): never grown or freed
     bool fixed_scratch = false;
@@ -174,6 +190,7 @@ struct pg_sim {
     double dt_last = 0.0;  // dt of the last integrating step
     int32_t integ = PG_INTEG_VERLET;
     double near = 0.0;  // near field in leaf widths (0: the reference's walk)
+    int64_t steps_known = -1;  // SegState.steps_done as last read back (-1: read it)
     double* stage = nullptr;   // euler / rk4: base state and rk4 sums (12 doubles per body)
     uint64_t stage_steps = 0;  // steps taken by the euler / rk4 stage loop
 };
@@ -222,6 +239,11 @@ extern "C" uint64_t pg_sim_bytes(uint64_t n, int32_t kind) {
 }
 
 // --------------------------------------------------------------- engine
+constexpr uint64_t kPinBytes = 64 << 10;    // pinned memory for tables and status, at first
+constexpr uint64_t kReturnBytes = 3 << 20;  // each half of the pinned memory states and results pass
+                                            // through (whole doubles)
+constexpr uint64_t kSmallCopy = 256 << 10;  // kernels read and write that memory in place up to here
+
 extern "C" int pg_engine_create(int device, uint64_t budget, pg_engine** out) {
     if (!out) return pg_set_error(PG_ERR_ARG, "out is NULL");
     int ndev = 0;
@@ -270,6 +292,10 @@ extern "C" void pg_engine_destroy(pg_engine* e) {
         (void)hipEventDestroy(ev.second.b);
     }
     (void)hipStreamDestroy(e->stream);
+    if (e->pin) (void)hipHostFree(e->pin);
+    if (e->ret) (void)hipHostFree(e->ret);
+    for (hipEvent_t ev : e->ret_ev)
+        if (ev) (void)hipEventDestroy(ev);
     delete e;
 }
 
@@ -515,6 +541,7 @@ static uint64_t carve_scratch(pg_engine* e, char* b, uint64_t bodies, uint64_t n
     e->ext_valid = 0;
     e->sorted_valid = 0;
     e->last_sim = nullptr;
+    e->up_kind = -1;
     return off;
 }
 
@@ -901,10 +928,197 @@ static int err_text(uint32_t bits) {
     }
 }
 
+// Pinned memory of at least `bytes`; what it held before is not kept.
+static int ensure_pinned(pg_engine* e, uint64_t bytes) {
+    if (bytes <= e->pin_bytes) return PG_OK;
+    uint64_t want = std::max(e->pin_bytes, kPinBytes);
+    while (want < bytes) want *= 2;
+    if (e->pin) HIP_TRY(hipStreamSynchronize(e->stream));
+    char* p = nullptr;
+    if (hipHostMalloc((void**)&p, want, hipHostMallocDefault) != hipSuccess)
+        return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)", (unsigned long long)want);
+    if (e->pin) (void)hipHostFree(e->pin);
+    e->pin = p;
+    e->pin_bytes = want;
+    return PG_OK;
+}
+
+// The device tables of the batch in e->h_*: nothing where they hold it
+// already (the same descriptors, or the same with the parities changed over,
+// *parity then 1); a batch of one segment writes them from its descriptors, a
+// larger one through pinned memory.
+static int upload_tables(pg_engine* e, const BatchPlan& bp, int* parity) {
+    const uint64_t bytes = bp.nseg * sizeof(SegDesc);
+    auto same = [&](int a, int b) {
+        return e->up_desc[a].size() == bp.nseg &&
+               memcmp(e->up_desc[a].data(), e->h_desc[b].data(), bytes) == 0;
+    };
+    *parity = 0;
+    if (e->up_kind == bp.kind && e->up_prec == bp.precision) {
+        if (same(0, 0) && same(1, 1)) return PG_OK;
+        if (same(0, 1) && same(1, 0)) {
+            *parity = 1;
+            return PG_OK;
+        }
+    }
+    e->up_kind = -1;
+    if (bp.nseg == 1) {
+        OneSegment a;
+        a.d[0] = e->h_desc[0][0];
+        a.d[1] = e->h_desc[1][0];
+        a.nchunks = bp.nchunks;
+        a.ntiles = bp.ntiles;
+        a.nblocks = bp.nblocks;
+        const uint32_t most = std::max(std::max(bp.nchunks, bp.ntiles + 1), bp.nblocks);
+        k_one_segment<<<(most + kBlock - 1) / kBlock, kBlock, 0, e->stream>>>(
+            a, e->desc[0], e->desc[1], e->seg_off, e->ext_seg, e->ext_chunk, e->tile_start,
+            e->blk_seg, e->blk_tile);
+    } else {
+        TableCopy c;
+        const void* src[kTables] = {e->h_desc[0].data(), e->h_desc[1].data(), e->h_seg_off.data(),
+                                    e->h_ext_seg.data(), e->h_ext_chunk.data(),
+                                    e->h_tile_start.data(), e->h_blk_seg.data(),
+                                    e->h_blk_tile.data()};
+        void* dst[kTables] = {e->desc[0], e->desc[1], e->seg_off, e->ext_seg,
+                              e->ext_chunk, e->tile_start, e->blk_seg, e->blk_tile};
+        const uint64_t len[kTables] = {bytes, bytes, (bp.nseg + 1) * 8ull, bp.nchunks * 4ull,
+                                       bp.nchunks * 4ull, (bp.ntiles + 1) * 4ull,
+                                       bp.nblocks * 4ull, bp.nblocks * 4ull};
+        const uint64_t head = align256((bp.nseg + 1) * sizeof(SegStatus));
+        uint64_t all = 0;
+        for (int t = 0; t < kTables; ++t) all += len[t];
+        PG_TRY(ensure_pinned(e, head + all));
+        if (e->pin_busy) HIP_TRY(hipStreamSynchronize(e->stream));
+        e->pin_busy = true;
+        char* to = e->pin + head;
+        c.src = (const uint32_t*)to;
+        for (int t = 0; t < kTables; ++t) {
+            if (len[t]) memcpy(to, src[t], len[t]);
+            to += len[t];
+            c.dst[t] = (uint32_t*)dst[t];
+            c.words[t] = (uint32_t)(len[t] / 4);
+        }
+        k_tables<<<grid_for(all / 4, 64), kBlock, 0, e->stream>>>(c);
+    }
+    HIP_TRY(hipGetLastError());
+    for (int q = 0; q < 2; ++q) e->up_desc[q] = e->h_desc[q];
+    e->up_kind = bp.kind;
+    e->up_prec = bp.precision;
+    return PG_OK;
+}
+
+// Asks for the status of the batch just enqueued (pinned memory, after
+// everything before it on the stream), and for the first `words` doubles of
+// its accelerations (at e->ret).
+static int enqueue_status(pg_engine* e, uint32_t nseg, uint32_t words = 0) {
+    PG_TRY(ensure_pinned(e, (nseg + 1) * sizeof(SegStatus)));
+    k_status<<<grid_for(std::max(nseg, words), 1u << 30), kBlock, 0, e->stream>>>(
+        e->desc[0], nseg, e->err_global, (SegStatus*)e->pin, e->acc_out, (double*)e->ret, words);
+    HIP_TRY(hipGetLastError());
+    e->pending = nseg;
+    return PG_OK;
+}
+
+// Waits for the stream and returns what the batch of e->h_sims reported.
+static int finish_batch(pg_engine* e) {
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    e->pin_busy = false;
+    if (e->profiling) ev_collect(e);
+    const SegStatus* st = (const SegStatus*)e->pin;
+    int rc = st[0].err ? err_text(st[0].err) : PG_OK;
+    for (uint64_t s = 0; s < e->pending; ++s) {
+        e->h_sims[s]->steps_known = st[1 + s].steps;
+        if (st[1 + s].err && rc == PG_OK) rc = err_text(st[1 + s].err);
+    }
+    e->pending = 0;
+    return rc;
+}
+
+// Pageable memory goes through two pinned halves, one on its way while the CPU
+// copies the other: the runtime's own copy pins or stages the caller's pages
+// first (590 KB up: 253 us against 43; 24 MB: 684 against 627), and for a
+// large fresh output array their faults cost more than the copy.
+
+// The halves, large enough for `bytes` at a time or of kReturnBytes.
+static int ensure_halves(pg_engine* e, uint64_t bytes) {
+    const uint64_t half = bytes <= kSmallCopy ? kSmallCopy : kReturnBytes;
+    if (e->ret_half >= half) return PG_OK;
+    for (hipEvent_t& ev : e->ret_ev)
+        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    char* p = nullptr;
+    if (hipHostMalloc((void**)&p, 2 * half, hipHostMallocDefault) != hipSuccess)
+        return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)", (unsigned long long)(2 * half));
+    if (e->ret) (void)hipHostFree(e->ret);
+    e->ret = p;
+    e->ret_half = half;
+    return PG_OK;
+}
+
+// A state of at most kSmallCopy bytes is read in place by the kernel that
+// unpacks it (*src then pinned memory), a larger one copied to `to`.
+static int copy_in(pg_engine* e, void* to, const void* from, uint64_t bytes, const void** src) {
+    PG_TRY(ensure_halves(e, bytes));
+    if (bytes <= kSmallCopy) {
+        memcpy(e->ret, from, bytes);
+        *src = e->ret;
+        return PG_OK;
+    }
+    *src = to;
+    for (uint64_t at = 0, c = 0; at < bytes; at += e->ret_half, ++c) {
+        const uint64_t len = std::min(e->ret_half, bytes - at);
+        char* half = e->ret + (c & 1) * e->ret_half;
+        if (c >= 2) HIP_TRY(hipEventSynchronize(e->ret_ev[c & 1]));
+        memcpy(half, (const char*)from + at, len);
+        HIP_TRY(hipMemcpyAsync((char*)to + at, half, len, hipMemcpyHostToDevice, e->stream));
+        HIP_TRY(hipEventRecord(e->ret_ev[c & 1], e->stream));
+    }
+    return PG_OK;
+}
+
+// Asks for the c-th chunk of `bytes` at device address src.
+static int fetch_chunk(pg_engine* e, const void* src, uint64_t bytes, uint64_t c) {
+    const uint64_t at = c * e->ret_half, len = std::min(e->ret_half, bytes - at);
+    HIP_TRY(hipMemcpyAsync(e->ret + (c & 1) * e->ret_half, (const char*)src + at, len,
+                           hipMemcpyDeviceToHost, e->stream));
+    HIP_TRY(hipEventRecord(e->ret_ev[c & 1], e->stream));
+    return PG_OK;
+}
+
+// take(offset, chunk, length) over `bytes` at device address src, in order;
+// the first chunk is asked for already.
+template <class Take>
+static int copy_back(pg_engine* e, const void* src, uint64_t bytes, Take take) {
+    const uint64_t chunks = (bytes + e->ret_half - 1) / e->ret_half;
+    for (uint64_t c = 0; c < chunks; ++c) {
+        if (c + 1 < chunks) PG_TRY(fetch_chunk(e, src, bytes, c + 1));
+        HIP_TRY(hipEventSynchronize(e->ret_ev[c & 1]));
+        const uint64_t at = c * e->ret_half;
+        take(at, e->ret + (c & 1) * e->ret_half, std::min(e->ret_half, bytes - at));
+    }
+    return PG_OK;
+}
+static int copy_out(pg_engine* e, const void* src, uint64_t bytes, void* out) {
+    if (!bytes) return PG_OK;
+    PG_TRY(ensure_halves(e, bytes));
+    PG_TRY(fetch_chunk(e, src, bytes, 0));
+#ifdef MADV_POPULATE_WRITE
+    // a fresh output's pages in one call, not one fault each (83 MB in 64
+    // arrays: 17 ms in all, 25 without)
+    const uintptr_t page = 4096, p0 = ((uintptr_t)out + page - 1) & ~(page - 1),
+                    p1 = ((uintptr_t)out + bytes) & ~(page - 1);
+    if (p1 > p0 + 16 * page) (void)madvise((void*)p0, p1 - p0, MADV_POPULATE_WRITE);
+#endif
+    return copy_back(e, src, bytes, [&](uint64_t at, const char* from, uint64_t len) {
+        memcpy((char*)out + at, from, len);
+    });
+}
+
 // Core of every device computation: `steps` steps of all sims together
-// (integrate) or one force evaluation into e->acc_out (no integrate).
+// (integrate) or one force evaluation into e->acc_out (no integrate). With
+// `wait` false the caller asks for the status and calls finish_batch.
 static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint32_t steps,
-                     bool integrate) {
+                     bool integrate, bool wait = true) {
     std::vector<pg_sim*>& sims = e->h_sims;
     sims.clear();
     for (uint32_t i = 0; i < count; ++i) {
@@ -915,6 +1129,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
         if (s->n) sims.push_back(s);
     }
     if (sims.empty() || steps == 0) return PG_OK;
+    for (pg_sim* s : sims) s->steps_known = -1;  // (finish_batch)
     BatchPlan bp;
     bp.kind = sims[0]->p.kind;
     bp.precision = sims[0]->p.precision;
@@ -1049,24 +1264,8 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
         off += sm->n;
     }
     e->h_seg_off[bp.nseg] = off;
-    HIP_TRY(hipMemcpyAsync(e->desc[0], e->h_desc[0].data(), bp.nseg * sizeof(SegDesc),
-                           hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipMemcpyAsync(e->desc[1], e->h_desc[1].data(), bp.nseg * sizeof(SegDesc),
-                           hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipMemcpyAsync(e->seg_off, e->h_seg_off.data(), (bp.nseg + 1) * 8,
-                           hipMemcpyHostToDevice, e->stream));
-    if (bp.nblocks) {
-        HIP_TRY(hipMemcpyAsync(e->blk_seg, e->h_blk_seg.data(), bp.nblocks * 4,
-                               hipMemcpyHostToDevice, e->stream));
-        HIP_TRY(hipMemcpyAsync(e->blk_tile, e->h_blk_tile.data(), bp.nblocks * 4,
-                               hipMemcpyHostToDevice, e->stream));
-    }
-    HIP_TRY(hipMemcpyAsync(e->ext_seg, e->h_ext_seg.data(), bp.nchunks * 4,
-                           hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipMemcpyAsync(e->ext_chunk, e->h_ext_chunk.data(), bp.nchunks * 4,
-                           hipMemcpyHostToDevice, e->stream));
-    HIP_TRY(hipMemcpyAsync(e->tile_start, e->h_tile_start.data(), (bp.ntiles + 1) * 4,
-                           hipMemcpyHostToDevice, e->stream));
+    int parity = 0;
+    PG_TRY(upload_tables(e, bp, &parity));
 
     // the batch's identity for the sample sort: its splitters may come from
     // the keys its previous step sorted only when the same batch ran last
@@ -1099,8 +1298,8 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     const bool warm_needs_sort = tree && bp.buckets;
     auto warm = [&] { return !tree || (ext_ok && (srt_ok || !warm_needs_sort)); };
     if (integrate && e->graphs && !e->profiling && steps >= 4 && !warm()) {
-        enqueue_step(e, bp, 0, false, !ext_ok, srt_ok);
-        enqueue_step(e, bp, 1, false, false, warm_needs_sort);
+        enqueue_step(e, bp, parity, false, !ext_ok, srt_ok);
+        enqueue_step(e, bp, parity ^ 1, false, false, warm_needs_sort);
         done = 2;
         ext_ok = true;
         srt_ok = warm_needs_sort;
@@ -1114,14 +1313,15 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
             sig.push_back((uint64_t)(uintptr_t)s);
             sig.push_back(s->n * 4 + (uint64_t)s->cur * 2 + (s->counting ? 1 : 0));
         }
+        sig.push_back((uint64_t)parity);
         hipGraphExec_t exec = nullptr;
         for (auto& g : e->graph_cache)
             if (g.sig == sig) exec = g.exec;
         if (!exec) {
             hipGraph_t graph = nullptr;
             HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-            enqueue_step(e, bp, 0, true, false, warm_needs_sort);
-            enqueue_step(e, bp, 1, true, false, warm_needs_sort);
+            enqueue_step(e, bp, parity, true, false, warm_needs_sort);
+            enqueue_step(e, bp, parity ^ 1, true, false, warm_needs_sort);
             HIP_TRY(hipStreamEndCapture(e->stream, &graph));
             HIP_TRY(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
             (void)hipGraphDestroy(graph);
@@ -1134,7 +1334,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
         for (; done + 2 <= steps; done += 2) HIP_TRY(hipGraphLaunch(exec, e->stream));
     }
     for (; done < steps; ++done) {
-        enqueue_step(e, bp, (int)(done & 1), false, !ext_ok, srt_ok);
+        enqueue_step(e, bp, (int)(done & 1) ^ parity, false, !ext_ok, srt_ok);
         ext_ok = true;
         srt_ok = warm_needs_sort;
         if (!integrate) break;
@@ -1142,8 +1342,6 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     e->ext_valid = integrate && tree ? bp.sort_tag : 0;
     e->sorted_valid = warm_needs_sort ? bp.sort_tag : 0;
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    if (e->profiling) ev_collect(e);
 
     if (flips && (steps & 1))
         for (pg_sim* s : sims) s->cur ^= 1;
@@ -1155,21 +1353,9 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     e->last_sorted = bp.buckets ? 1 : bp.passes & 1;
     e->last_dim = bp.dim;
     e->last_lmax = bp.lmax;
-
-    uint32_t gerr = 0;
-    HIP_TRY(hipMemcpy(&gerr, e->err_global, 4, hipMemcpyDeviceToHost));
-    if (gerr) {
-        uint32_t z = 0;
-        HIP_TRY(hipMemcpy(e->err_global, &z, 4, hipMemcpyHostToDevice));
-        return err_text(gerr);
-    }
-    int rc = PG_OK;
-    for (pg_sim* s : sims) {
-        SegState st;
-        HIP_TRY(hipMemcpy(&st, s->st, sizeof st, hipMemcpyDeviceToHost));
-        if (st.err && rc == PG_OK) rc = err_text(st.err);
-    }
-    return rc;
+    if (!wait) return PG_OK;
+    PG_TRY(enqueue_status(e, bp.nseg));
+    return finish_batch(e);
 }
 
 // ------------------------------------------------------------- simulations
@@ -1279,7 +1465,9 @@ extern "C" int pg_sim_set_counting(pg_sim* s, int enable) {
     return PG_OK;
 }
 
-extern "C" int pg_sim_upload(pg_sim* s, const Entity* state, uint64_t n) {
+// pg_sim_upload without the wait for the stream: the pinned halves hold (part
+// of) the state until then.
+static int upload_async(pg_sim* s, const Entity* state, uint64_t n) {
     if (!s) return pg_set_error(PG_ERR_ARG, "sim is NULL");
     if (n != s->n) return pg_set_error(PG_ERR_ARG, "n %llu != sim n %llu", (unsigned long long)n,
                                        (unsigned long long)s->n);
@@ -1289,19 +1477,29 @@ extern "C" int pg_sim_upload(pg_sim* s, const Entity* state, uint64_t n) {
     HIP_TRY(hipSetDevice(e->device));
     s->cur = 0;
     if (n) {
-        HIP_TRY(hipMemcpyAsync(s->aos, state, n * sizeof(Entity), hipMemcpyHostToDevice, e->stream));
-        k_unpack<<<grid_for(n, 1u << 30), kBlock, 0, e->stream>>>(
-            s->aos, n, s->pos[0], s->prv[0], s->vx[0], s->vy[0], s->vz[0]);
+        const void* src = nullptr;
+        PG_TRY(copy_in(e, s->aos, state, n * sizeof(Entity), &src));
+        k_unpack<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, e->stream>>>(
+            (const uint64_t*)src, src == s->aos ? nullptr : (uint64_t*)s->aos, n, s->pos[0], s->prv[0], s->vx[0], s->vy[0], s->vz[0], s->st,
+            e->sc ? &e->sc->ext_tag : nullptr);
         HIP_TRY(hipGetLastError());
+    } else {
+        HIP_TRY(hipMemsetAsync(s->st, 0, sizeof(SegState), e->stream));
     }
-    HIP_TRY(hipMemsetAsync(s->st, 0, sizeof(SegState), e->stream));
     s->stage_steps = 0;
+    s->steps_known = 0;
     // new positions: no extent partials are current
-    if (e->sc) HIP_TRY(hipMemsetAsync(&e->sc->ext_tag, 0, sizeof(uint64_t), e->stream));
     e->ext_valid = 0;
-    HIP_TRY(hipStreamSynchronize(e->stream));
     s->uploaded = true;
     if (e->last_sim == s) e->last_sim = nullptr;
+    return PG_OK;
+}
+
+extern "C" int pg_sim_upload(pg_sim* s, const Entity* state, uint64_t n) {
+    if (!s) return pg_set_error(PG_ERR_ARG, "sim is NULL");
+    std::lock_guard<std::recursive_mutex> lk(s->eng->mu);
+    PG_TRY(upload_async(s, state, n));
+    HIP_TRY(hipStreamSynchronize(s->eng->stream));
     return PG_OK;
 }
 
@@ -1324,6 +1522,7 @@ extern "C" int pg_sim_upload_state(pg_sim* s, const Entity* state, const Entity*
     memset(&st, 0, sizeof st);
     st.steps_done = 1;
     HIP_TRY(hipMemcpyAsync(s->st, &st, sizeof st, hipMemcpyHostToDevice, e->stream));
+    s->steps_known = 1;
     HIP_TRY(hipStreamSynchronize(e->stream));
     return PG_OK;
 }
@@ -1331,12 +1530,15 @@ extern "C" int pg_sim_upload_state(pg_sim* s, const Entity* state, const Entity*
 // Where the current state's velocities come from: the stored arrays up to and
 // right after the Taylor first step, the backward difference afterwards.
 static int velocity_source(pg_sim* s, VelocitySource* vs) {
-    SegState st;
-    HIP_TRY(hipMemcpy(&st, s->st, sizeof st, hipMemcpyDeviceToHost));
+    if (s->steps_known < 0) {
+        SegState st;
+        HIP_TRY(hipMemcpy(&st, s->st, sizeof st, hipMemcpyDeviceToHost));
+        s->steps_known = (int64_t)std::min<uint64_t>(st.steps_done, 0xFFFFFFFFu);
+    }
     const int c = s->cur;
     vs->vx = s->vx[c]; vs->vy = s->vy[c]; vs->vz = s->vz[c];
     vs->prv = s->prv[c];
-    vs->derive = s->integ == PG_INTEG_VERLET && st.steps_done >= 2 ? 1 : 0;
+    vs->derive = s->integ == PG_INTEG_VERLET && s->steps_known >= 2 ? 1 : 0;
     vs->dt = s->dt_last;
     return PG_OK;
 }
@@ -1355,14 +1557,13 @@ extern "C" int pg_sim_download(pg_sim* s, Entity* out, uint64_t n) {
     PG_TRY(velocity_source(s, &vs));
     k_pack<<<grid_for(n, 1u << 30), kBlock, 0, e->stream>>>(s->aos, n, s->pos[c], vs, s->prv[c]);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out, s->aos, n * sizeof(Entity), hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    return PG_OK;
+    return copy_out(e, s->aos, n * sizeof(Entity), out);
 }
 
 static StageState stage_state(pg_sim* s) {
     const int c = s->cur;
-    return StageState{s->pos[c], s->prv[c], s->vx[c], s->vy[c], s->vz[c], s->n};
+    return StageState{s->pos[c], s->prv[c], s->vx[c], s->vy[c], s->vz[c], s->n,
+                      s->st,     s->eng->err_global};
 }
 
 // euler.rs:17-49 / rk4.rs:24-182 on the device: each acceleration pass is
@@ -1377,23 +1578,26 @@ static int step_stages(pg_engine* e, pg_sim* s, uint32_t steps) {
     double* ksum = s->stage + 6 * s->n;
     for (uint32_t k = 0; k < steps; ++k) {
         if (s->integ == PG_INTEG_EULER) {
-            PG_TRY(run_batch(e, &s, 1, 1, false));
+            PG_TRY(run_batch(e, &s, 1, 1, false, false));
             k_euler_update<<<g, kBlock, 0, e->stream>>>(stage_state(s), e->acc_out, s->p.dt);
             HIP_TRY(hipGetLastError());
         } else {
             k_rk4_begin<<<g, kBlock, 0, e->stream>>>(stage_state(s), base);
             HIP_TRY(hipGetLastError());
             for (int st = 0; st < 4; ++st) {
-                PG_TRY(run_batch(e, &s, 1, 1, false));
+                PG_TRY(run_batch(e, &s, 1, 1, false, false));
                 k_rk4_stage<<<g, kBlock, 0, e->stream>>>(stage_state(s), e->acc_out, base, ksum,
                                                          s->p.dt, st);
                 HIP_TRY(hipGetLastError());
             }
         }
+        e->ext_valid = 0;  // the stage kernels moved the bodies
+        // one wait a step: where a pass failed on the device, its error bits
+        // are sticky and no later stage has changed the state
+        PG_TRY(enqueue_status(e, 1));
+        PG_TRY(finish_batch(e));
         s->stage_steps += 1;
     }
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    e->ext_valid = 0;  // the stage kernels moved the bodies
     return PG_OK;
 }
 
@@ -1465,6 +1669,7 @@ extern "C" int pg_sim_set_integrator(pg_sim* s, int32_t integrator) {
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemsetAsync(s->st, 0, sizeof(SegState), e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
+        s->steps_known = 0;
     }
     s->integ = integrator;
     return PG_OK;
@@ -1549,6 +1754,7 @@ extern "C" int pg_engine_autotune(pg_engine* e, pg_sim* const* sims, uint32_t co
             sims[i]->cur = saved[i].cur;
             sims[i]->stage_steps = saved[i].stage_steps;
             sims[i]->dt_last = saved[i].dt_last;
+            sims[i]->steps_known = -1;
         }
         // the positions changed under the extent partials the last walk left:
         // the device-side tag that lets the extent pass skip goes too (as on
@@ -1612,8 +1818,7 @@ extern "C" int pg_sim_accel(pg_sim* s, double* acc) {
     std::lock_guard<std::recursive_mutex> lk(e->mu);
     HIP_TRY(hipSetDevice(e->device));
     PG_TRY(run_batch(e, &s, 1, 1, false));
-    if (s->n) HIP_TRY(hipMemcpy(acc, e->acc_out, s->n * 24, hipMemcpyDeviceToHost));
-    return PG_OK;
+    return copy_out(e, e->acc_out, s->n * 24, acc);
 }
 
 extern "C" int pg_transform_aos(pg_engine* e, const pg_params* p, const Entity* state, uint64_t n,
@@ -1630,15 +1835,30 @@ extern "C" int pg_transform_aos(pg_engine* e, const pg_params* p, const Entity* 
     }
     if (!e->xform) PG_TRY(pg_sim_create(e, n, p, &e->xform));
     PG_TRY(pg_sim_set_params(e->xform, p));
-    PG_TRY(pg_sim_upload(e->xform, state, n));
-    std::vector<double> a(n * 3);
-    PG_TRY(pg_sim_accel(e->xform, a.data()));
-    for (uint64_t i = 0; i < n; ++i) {
-        acc[i].x += a[3 * i + 0];
-        acc[i].y += a[3 * i + 1];
-        acc[i].z += a[3 * i + 2];
+    // the state up, the pass, its status and the first accelerations back
+    // with one wait; few accelerations come with the status
+    const bool small = n * 24 <= kSmallCopy;
+    static_assert(sizeof(Acceleration) == 24, "accelerations as an array of doubles");
+    double* out = reinterpret_cast<double*>(acc);
+    int rc = upload_async(e->xform, state, n);
+    if (rc == PG_OK) rc = run_batch(e, &e->xform, 1, 1, false, false);
+    if (rc == PG_OK) rc = enqueue_status(e, 1, small ? (uint32_t)n * 3 : 0);
+    if (rc == PG_OK && !small) rc = fetch_chunk(e, e->acc_out, n * 24, 0);
+    if (rc != PG_OK) {
+        (void)hipStreamSynchronize(e->stream);  // the pinned halves are in use
+        return rc;
     }
-    return PG_OK;
+    PG_TRY(finish_batch(e));
+    if (small) {
+        const double* a = (const double*)e->ret;
+        for (uint64_t i = 0; i < n * 3; ++i) out[i] += a[i];
+        return PG_OK;
+    }
+    return copy_back(e, e->acc_out, n * 24, [&](uint64_t at, const char* from, uint64_t bytes) {
+        const double* a = (const double*)from;
+        double* o = out + at / 8;
+        for (uint64_t i = 0; i < bytes / 8; ++i) o[i] += a[i];
+    });
 }
 
 extern "C" int pg_sim_energy(pg_sim* s, double out[6]) {
@@ -1906,6 +2126,10 @@ static int noalloc_setup(NoAllocCtx& c, int device, hipStream_t stream) {
     e.h_tile0.reserve(1);
     e.h_desc[0].reserve(1);
     e.h_desc[1].reserve(1);
+    PG_TRY(ensure_pinned(&e, kPinBytes));
+    PG_TRY(ensure_halves(&e, kReturnBytes));
+    e.up_desc[0].reserve(1);
+    e.up_desc[1].reserve(1);
     e.h_seg_off.reserve(2);
     e.h_blk_seg.reserve(blocks);
     e.h_blk_tile.reserve(blocks);

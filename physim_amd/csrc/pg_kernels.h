@@ -3921,12 +3921,112 @@ __global__ __launch_bounds__(kBlock) void k_energy(const double4* __restrict__ p
         partial[5 * (blockIdx.y * gridDim.x + blockIdx.x) + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// AoS <-> SoA at the host boundary.
-__global__ void k_unpack(const Entity* __restrict__ aos, uint64_t n, double4* __restrict__ pos,
-                         double4* __restrict__ prv, double* vx, double* vy, double* vz) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The tables of a batch of one segment, from its descriptors (both parities)
+// passed by value: no copy from host memory for a call on one simulation. The
+// largest table's length of threads.
+struct OneSegment {
+    SegDesc d[2];
+    uint32_t nchunks, ntiles, nblocks;
+};
+__global__ __launch_bounds__(kBlock) void k_one_segment(
+    OneSegment a, SegDesc* __restrict__ d0, SegDesc* __restrict__ d1, uint64_t* __restrict__ seg_off,
+    uint32_t* __restrict__ ext_seg, uint32_t* __restrict__ ext_chunk,
+    uint32_t* __restrict__ tile_start, uint32_t* __restrict__ blk_seg,
+    uint32_t* __restrict__ blk_tile) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i == 0) {
+        *d0 = a.d[0];
+        *d1 = a.d[1];
+        seg_off[0] = 0;
+        seg_off[1] = a.d[0].n;
+    }
+    if (i < a.nchunks) {
+        ext_seg[i] = 0;
+        ext_chunk[i] = i;
+    }
+    if (i <= a.ntiles)
+        tile_start[i] = (uint32_t)min((uint64_t)i * kNodeTile, a.d[0].n);
+    if (i < a.nblocks) {
+        blk_seg[i] = 0;
+        blk_tile[i] = i / a.d[0].ngroup | (i % a.d[0].ngroup) << 24;
+    }
+}
+
+// The tables of a batch of several segments, packed one after another in
+// pinned host memory, to their places (32-bit words).
+constexpr int kTables = 8;
+struct TableCopy {
+    const uint32_t* src;
+    uint32_t* dst[kTables];
+    uint32_t words[kTables];
+};
+__global__ __launch_bounds__(kBlock) void k_tables(TableCopy c) {
+    const uint32_t* src = c.src;
+    for (int t = 0; t < kTables; ++t) {
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < c.words[t]; i += gridDim.x * kBlock)
+            c.dst[t][i] = src[i];
+        src += c.words[t];
+    }
+}
+
+// What a call reports, into pinned host memory: the batch-wide error bits
+// (cleared), then each segment's error bits and steps done. A small
+// transform's accelerations (`words` doubles) go with it, in place of a copy
+// of their own.
+struct SegStatus {
+    uint32_t err, steps;
+};
+__global__ __launch_bounds__(kBlock) void k_status(const SegDesc* __restrict__ desc, uint32_t nseg,
+                                                   uint32_t* __restrict__ err_global,
+                                                   SegStatus* __restrict__ out,
+                                                   const double* __restrict__ acc,
+                                                   double* __restrict__ acc_out, uint32_t words) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t == 0) {
+        out[0] = SegStatus{*err_global, 0u};
+        *err_global = 0;
+    }
+    if (t < nseg) {
+        const SegState* st = desc[t].st;
+        out[1 + t] = SegStatus{st->err, (uint32_t)min(st->steps_done, (uint64_t)0xFFFFFFFFu)};
+    }
+    if (t < words) acc_out[t] = acc[t];
+}
+
+// AoS <-> SoA at the host boundary. An upload also starts the simulation's
+// step state afresh, and no extent partials are current then (ext_tag; may be
+// NULL). A block takes its records in through LDS, word by word in order (a
+// thread reading its own 80-byte record asks for a line per lane and word), so
+// that `src` may be pinned host memory: a small state needs no copy of its own
+// (64 KB: 22 us against 44 for the runtime's pageable copy); it is kept in
+// `aos` then.
+constexpr int kEntityWords = sizeof(Entity) / 8;
+static_assert(sizeof(Entity) % 8 == 0, "records of whole 8-byte words");
+__global__ __launch_bounds__(kBlock) void k_unpack(
+    const uint64_t* __restrict__ src, uint64_t* __restrict__ aos, uint64_t n,
+    double4* __restrict__ pos, double4* __restrict__ prv, double* vx, double* vy, double* vz,
+    SegState* __restrict__ st, uint64_t* __restrict__ ext_tag) {
+    __shared__ uint64_t rec[kBlock * kEntityWords];
+    const uint64_t base = (uint64_t)blockIdx.x * kBlock, i = base + threadIdx.x;
+    const uint32_t words = (uint32_t)min((uint64_t)kBlock, n - base) * kEntityWords;
+    uint64_t v[kEntityWords];
+    for (int k = 0; k < kEntityWords; ++k) {
+        const uint32_t w = k * kBlock + threadIdx.x;
+        if (w < words) v[k] = src[base * kEntityWords + w];
+    }
+    for (int k = 0; k < kEntityWords; ++k) {
+        const uint32_t w = k * kBlock + threadIdx.x;
+        if (w >= words) break;
+        rec[w] = v[k];
+        if (aos) aos[base * kEntityWords + w] = v[k];
+    }
+    if (i == 0) {
+        *st = SegState{};
+        if (ext_tag) *ext_tag = 0;
+    }
+    __syncthreads();
     if (i >= n) return;
-    const Entity e = aos[i];
+    const Entity e = *(const Entity*)(rec + threadIdx.x * kEntityWords);
     pos[i] = make_double4(e.x, e.y, e.z, e.mass);
     prv[i] = make_double4(e.x, e.y, e.z, make_tag((uint32_t)i, e.fixed != 0));
     vx[i] = e.vx; vy[i] = e.vy; vz[i] = e.vz;
@@ -3989,13 +4089,21 @@ struct StageState {
     const double4* prv;  // the tags
     double *vx, *vy, *vz;
     uint64_t n;
+    const SegState* st;
+    const uint32_t* err_global;
 };
+
+// An acceleration pass has failed (sticky until it is reported): the state
+// stays as it is.
+__device__ __forceinline__ bool stage_failed(const StageState& s) {
+    return (s.st->err | *s.err_global) != 0;
+}
 
 // euler.rs:26-45: x' = x + v dt + 0.5 a dt^2 (dt.powi(2) = dt * dt),
 // v' = v + a dt, every body (fixed ones have a = 0 and keep moving).
 __global__ void k_euler_update(StageState st, const double* __restrict__ acc, double dt) {
     const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= st.n) return;
+    if (j >= st.n || stage_failed(st)) return;
     const double* a = acc + 3 * (uint64_t)tag_id(st.prv[j].w);
     const double dt2 = dt * dt;
     const double4 p = st.pos[j];
@@ -4029,7 +4137,7 @@ __global__ void k_rk4_stage(StageState st, const double* __restrict__ acc,
                             const double* __restrict__ base, double* __restrict__ ksum, double dt,
                             int stage) {
     const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= st.n) return;
+    if (j >= st.n || stage_failed(st)) return;
     const double4 pr = st.prv[j];
     const uint64_t u = tag_id(pr.w);
     const double* a = acc + 3 * u;
