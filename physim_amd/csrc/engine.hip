@@ -813,23 +813,31 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
             desc, e->tile_start, e->ext_partial, bp.nchunks, skeys, svals, bp.nseg, bp.segbits, bp.lmax, e->node_local,
             e->tile_tot, e->lo_level, e->lvl_first, e->deep, e->err_global, e->leaf_lv, e->leafpos);
     });
-    launch(e, cap, "tree_scan", [&] {
-        k_tree_scan<<<1 + kTopSlots, kScanThreads, 0, st>>>(e->tile_tot, e->tile_base, tiles,
-                                                             e->lvl_first, e->first_node, total,
-                                                             e->node_span, e->cap_nodes);
-    });
+    const bool few = tiles <= (unsigned)kFewTiles;
+    if (!few)
+        launch(e, cap, "tree_scan", [&] {
+            k_tree_scan<<<1 + kTopSlots, kScanThreads, 0, st>>>(e->tile_tot, e->tile_base, tiles,
+                                                                 e->lvl_first, e->first_node, total,
+                                                                 e->node_span, e->cap_nodes);
+        });
     launch(e, cap, "nodes", [&] {
-        k_nodes<DIM><<<tiles, kNodeThreads, 0, st>>>(
-            desc, e->seg_off, e->tile_start, total, skeys, bp.nseg, bp.segbits, bp.lmax,
-            e->node_local, e->tile_base, e->lvl_first, e->first_node, e->lo_level, e->hot,
-            e->cap_nodes, e->top_slot, e->top_last, e->out_part, e->in_part, e->tot_part, e->deep,
-            e->sc, e->leafpos, e->node_span);
+#define PG_NODES(FEW)                                                                          \
+    k_nodes<DIM, FEW><<<tiles, kNodeThreads, 0, st>>>(                                         \
+        desc, e->seg_off, e->tile_start, total, skeys, bp.nseg, bp.segbits, bp.lmax,          \
+        e->node_local, e->tile_tot, e->tile_base, e->lvl_first, e->first_node, e->lo_level,   \
+        e->hot, e->cap_nodes, e->top_slot, e->top_last, e->out_part, e->in_part, e->tot_part, \
+        e->deep, e->sc, e->leafpos, e->node_span)
+        if (few) PG_NODES(true);
+        else PG_NODES(false);
+#undef PG_NODES
     });
-    launch(e, cap, "com_span", [&] {
-        k_com_span<<<dim3(tiles, kComSpanGroups), kBlock, 0, st>>>(
-            desc, e->seg_off, bp.nseg, e->tile_start, e->hot, e->top_last, e->top_slot,
-            e->out_part, e->in_part, e->tot_part, e->sc);
-    });
+    // (no node spans tiles where every segment is one)
+    if (tiles > bp.nseg)
+        launch(e, cap, "com_span", [&] {
+            k_com_span<<<dim3(tiles, kComSpanGroups), kBlock, 0, st>>>(
+                desc, e->seg_off, bp.nseg, e->tile_start, e->hot, e->top_last, e->top_slot,
+                e->out_part, e->in_part, e->tot_part, e->sc);
+        });
     launch(e, cap, "walk", [&] {
 #define PG_WALK(NEAR, COUNT)                                                                   \
     k_walk<DIM, FP64, INTEG, NEAR, COUNT><<<grid_for(total, 1u << 30), kBlock, 0, st>>>(       \

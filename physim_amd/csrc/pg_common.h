@@ -35,6 +35,7 @@ constexpr int kNodeTile = 1024;    // sorted bodies per node-building block
 constexpr int kNodeThreads = 512;  // threads per node-building block (two bodies each)
 constexpr int kNodeLds = 1792;     // kNodeTile bodies + up to kNodeLds - kNodeTile internal nodes: built one
                                    // node per thread (more internal nodes: body by body)
+constexpr int kFewTiles = 64;      // batches of at most this many node tiles: no scan over the tiles apart
 constexpr int kTopSlots = 65;      // tree levels 0..64: one tile-spanning node each
 constexpr int kMaxTieRun = 256;    // longest run of equal keys ordered by their deep keys
 constexpr int kMaxLcp = 64;        // deepest common prefix, in levels, of two bodies: the

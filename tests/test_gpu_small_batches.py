@@ -1,0 +1,36 @@
+"""Launches that only large batches need: a system stepped alone (few node
+tiles, its own sort) against the same system stepped beside a filler that
+takes the batch past every such line. The tree, the order and the arithmetic
+do not depend on it: every bit is compared."""
+import numpy as np
+import pytest
+
+import physim_amd as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def filler():
+    return P.gen_plummer_virial(150000, seed=1, mass=1.0, a=0.1)
+
+
+@pytest.mark.parametrize("kind", ["astro2", "astro"])
+@pytest.mark.parametrize("model", ["cube", "plummer"])
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 513, 1024, 1025, 2049, 8193, 16384, 16385, 65535,
+                               65536, 65537])
+def test_alone_equals_beside_a_large_one(engine, filler, kind, model, n):
+    if model == "cube" and n > 2:
+        s = P.cube_and_stars(n - 2, seed=n)
+    else:
+        s = P.gen_plummer_virial(n, seed=n, mass=1.0, a=0.1)
+    assert len(s) == n
+    kw = dict(kind=kind, theta=0.9, e=0.05, dt=1e-4)
+    alone, beside, big = (P.Sim(engine, x, **kw) for x in (s, s, filler))
+    alone.step(7)
+    engine.batch_step([beside, big], 7)
+    assert alone.download().tobytes() == beside.download().tobytes()
+    a = alone.accel()
+    assert a.tobytes() == beside.accel().tobytes()
+    for x in (alone, beside, big):
+        x.close()
