@@ -33,8 +33,11 @@ constexpr int kExtentChunk = 4096; // bodies per extent partial
 constexpr uint32_t kExtentBlocks = 256;  // blocks of the extent pass (each takes chunks in turn)
 constexpr int kNodeTile = 1024;    // sorted bodies per node-building block
 constexpr int kNodeThreads = 512;  // threads per node-building block (two bodies each)
-constexpr int kNodeLds = 1792;     // kNodeTile bodies + up to kNodeLds - kNodeTile internal nodes: built one
-                                   // node per thread (more internal nodes: body by body)
+constexpr int kNodeLds = 2016;     // kNodeTile bodies + up to kNodeLds - kNodeTile internal nodes: built one
+                                   // node per thread (more internal nodes: body by body). Uniform
+                                   // quadtrees have 0.7 per body, up to 0.9 in a tile: with a list of
+                                   // 768 a build of 50,003 bodies took 34 us, with 992 (the most at
+                                   // three blocks a CU) 21
 constexpr int kFewTiles = 64;      // batches of at most this many node tiles: no scan over the tiles apart
 constexpr int kTopSlots = 65;      // tree levels 0..64: one tile-spanning node each
 constexpr int kMaxTieRun = 256;    // longest run of equal keys ordered by their deep keys

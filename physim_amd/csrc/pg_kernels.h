@@ -838,8 +838,10 @@ __device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t total,
         const double4 q = d.spos[src];
         const double px = q.x, py = q.y, pz = q.z;
         double ext = E, cx = 0.0, cy = 0.0, cz = 0.0;
-        DeepKey dk;
-        for (int i = 0; i < kDeepWords; ++i) dk.w[i] = 0;
+        // (words chosen, not indexed, here and in descend: an indexed record
+        // lives in scratch, and kernels with scratch start later)
+        static_assert(kDeepWords == 3, "three words");
+        uint64_t w0 = 0, w1 = 0, w2 = 0;
         for (int l = 0; l < deepest; ++l) {
             uint32_t o = (uint32_t)(px > cx) | ((uint32_t)(py > cy) << 1);
             if (DIM == 3) o |= (uint32_t)(pz > cz) << 2;
@@ -850,10 +852,13 @@ __device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t total,
             ext = h2;
             if (l >= lmax) {
                 const int t = l - lmax;
-                dk.w[t / W] |= (uint64_t)o << (DIM * (W - 1 - t % W));
+                const uint64_t dig = (uint64_t)o << (DIM * (W - 1 - t % W));
+                w0 |= t < W ? dig : 0ull;
+                w1 |= t >= W && t < 2 * W ? dig : 0ull;
+                w2 |= t >= 2 * W ? dig : 0ull;
             }
         }
-        deep[j] = dk;
+        deep[j] = DeepKey{{w0, w1, w2}};
     }
     for (uint64_t j = g + 1; j <= r; ++j) {
         const DeepKey kv = deep[j];
@@ -1931,7 +1936,7 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
         __syncthreads();
         if (slots) {
             // only the heads the slot sort marked start runs of equal keys
-#pragma unroll
+#pragma unroll 1
             for (int e = 0; e < 4; ++e)
                 if ((heads >> e) & 1u)
                     order_tie_run<DIM>(desc, total, keys, vals, deep, nseg, segbits, lmax,
@@ -2429,10 +2434,12 @@ __device__ __forceinline__ void descend(uint64_t key, const DeepKey& dk, int lma
     const int a = min(to, lmax);
     if (from < a) descend_w<DIM>(~key << (64 - DIM * (lmax - from)), a - from, ext, cx, cy, cz);
     constexpr int W = kWordLevels<DIM>;
+    const uint64_t w0 = dk.w[0], w1 = dk.w[1], w2 = dk.w[2];
     for (int l = max(from, lmax); l < to;) {
         const int t = l - lmax, p = t % W;
         const int n = min(to - l, W - p);
-        descend_w<DIM>(~dk.w[t / W] << (64 - DIM * (W - p)), n, ext, cx, cy, cz);
+        const uint64_t w = t < W ? w0 : t < 2 * W ? w1 : w2;
+        descend_w<DIM>(~w << (64 - DIM * (W - p)), n, ext, cx, cy, cz);
         l += n;
     }
 }

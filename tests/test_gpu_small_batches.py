@@ -34,3 +34,23 @@ def test_alone_equals_beside_a_large_one(engine, filler, kind, model, n):
     assert a.tobytes() == beside.accel().tobytes()
     for x in (alone, beside, big):
         x.close()
+
+
+@pytest.mark.parametrize("pairs", [0, 20, 30, 36, 42, 60])
+def test_tiles_around_the_node_list(engine, pairs):
+    """One node tile of a quadtree whose internal nodes go from 0.7 to 1.2 per
+    body: up to 992 are built one per thread, more body by body."""
+    from oracle import oracle as O
+
+    rng = np.random.default_rng(pairs)
+    s = np.zeros(1024, P.ENTITY)
+    for f in "xyz":
+        s[f] = rng.uniform(-1.0, 1.0, len(s))
+    for f in "xy":  # (bodies near another: a chain of cells each)
+        s[f][:pairs] = s[f][512:512 + pairs] + rng.uniform(1e-4, 2e-4, pairs)
+    s["mass"] = rng.uniform(0.5, 1.5, len(s))
+    ref, _, fault = O.bh_transform(s, 0.7, 0.1, 2)
+    assert fault == 0
+    a = P.Sim(engine, s, kind="astro", theta=0.7, e=0.1, precision="fp64").accel()
+    r = np.linalg.norm(a - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert np.quantile(r, 0.99) <= 1e-11 and r.max() <= 1e-8
