@@ -794,6 +794,28 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
     }
 }
 
+// The reference's descent to a cell (child centres, octree.rs:160-215 /
+// quadtree.rs:161-194):
+// n levels down from a cell of half-width ext and centre c, the half-width
+// halves and the centre moves by it along each axis, up where the key's
+// octant bit is set, else down. w holds the digits to follow inverted and
+// left-aligned (the next digit's DIM bits on top, x lowest), so a digit's
+// inverted bit is the sign of that axis' move; c + (-h) is c - h exactly.
+template <int DIM>
+__device__ __forceinline__ void descend_w(uint64_t w, int n, double& ext, double& cx, double& cy,
+                                          double& cz) {
+    for (int l = 0; l < n; ++l) {
+        const uint32_t top = (uint32_t)(w >> 32);
+        ext = half(ext);
+        const uint64_t hb = f64_bits(ext);
+        const uint32_t lo = (uint32_t)hb, hi = (uint32_t)(hb >> 32);
+        cx += __hiloint2double((int)(hi | ((top << (DIM - 1)) & 0x80000000u)), (int)lo);
+        cy += __hiloint2double((int)(hi | ((top << (DIM - 2)) & 0x80000000u)), (int)lo);
+        if (DIM == 3) cz += __hiloint2double((int)(hi | (top & 0x80000000u)), (int)lo);
+        w <<= DIM;
+    }
+}
+
 // The reference's tree keeps splitting bodies that share every level a key
 // holds (octree.rs:92-125, down to depth 64). After the sort, each run of
 // equal keys (in practice two or three bodies of a dense core) gets the
@@ -804,9 +826,39 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
 template <int DIM>
 __device__ __forceinline__ bool deep_less(const DeepKey& a, uint32_t va, const DeepKey& b,
                                           uint32_t vb) {
-    for (int i = 0; i < kDeepWords; ++i)
-        if (a.w[i] != b.w[i]) return a.w[i] < b.w[i];
-    return va < vb;
+    static_assert(kDeepWords == 3, "three words");
+    return a.w[0] != b.w[0]   ? a.w[0] < b.w[0]
+           : a.w[1] != b.w[1] ? a.w[1] < b.w[1]
+           : a.w[2] != b.w[2] ? a.w[2] < b.w[2]
+                              : va < vb;
+}
+// The deep key of the body at q with first word `key` in a segment of extent
+// E: its descent from level lmax down to the first no two bodies may share.
+template <int DIM>
+__device__ __forceinline__ DeepKey deep_key(uint64_t key, double4 q, double E, int lmax) {
+    static_assert(kDeepWords == 3, "three words");
+    constexpr int W = kWordLevels<DIM>;
+    const int deepest = min(kMaxLcp + 1, lmax + kDeepWords * W);
+    double ext = E, cx = 0.0, cy = 0.0, cz = 0.0;
+    descend_w<DIM>(~key << (64 - DIM * lmax), lmax, ext, cx, cy, cz);
+    // (words chosen, not indexed, here and in descend: an indexed record
+    // lives in scratch, and kernels with scratch start later)
+    uint64_t w0 = 0, w1 = 0, w2 = 0;
+    for (int l = lmax; l < deepest; ++l) {
+        uint32_t o = (uint32_t)(q.x > cx) | ((uint32_t)(q.y > cy) << 1);
+        if (DIM == 3) o |= (uint32_t)(q.z > cz) << 2;
+        const double h2 = half(ext);
+        cx = (o & 1u) ? cx + h2 : cx - h2;
+        cy = (o & 2u) ? cy + h2 : cy - h2;
+        if (DIM == 3) cz = (o & 4u) ? cz + h2 : cz - h2;
+        ext = h2;
+        const int t = l - lmax;
+        const uint64_t dig = (uint64_t)o << (DIM * (W - 1 - t % W));
+        w0 |= t < W ? dig : 0ull;
+        w1 |= t >= W && t < 2 * W ? dig : 0ull;
+        w2 |= t >= 2 * W ? dig : 0ull;
+    }
+    return DeepKey{{w0, w1, w2}};
 }
 template <int DIM>
 __device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t total,
@@ -826,39 +878,13 @@ __device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t total,
         return;
     }
     const double E = bits_f64(d.st->extent_bits);
-    constexpr int W = kWordLevels<DIM>;
-    // the descent down to the first level no two bodies may share
-    const int deepest = min(kMaxLcp + 1, lmax + kDeepWords * W);
     for (uint64_t j = g; j <= r; ++j) {
         const uint64_t src = (uint64_t)svals[j] - d.off;
         if (src >= d.n) {
             atomicOr(&d.st->err, kErrCapacity);
             return;
         }
-        const double4 q = d.spos[src];
-        const double px = q.x, py = q.y, pz = q.z;
-        double ext = E, cx = 0.0, cy = 0.0, cz = 0.0;
-        // (words chosen, not indexed, here and in descend: an indexed record
-        // lives in scratch, and kernels with scratch start later)
-        static_assert(kDeepWords == 3, "three words");
-        uint64_t w0 = 0, w1 = 0, w2 = 0;
-        for (int l = 0; l < deepest; ++l) {
-            uint32_t o = (uint32_t)(px > cx) | ((uint32_t)(py > cy) << 1);
-            if (DIM == 3) o |= (uint32_t)(pz > cz) << 2;
-            const double h2 = half(ext);
-            cx = (o & 1u) ? cx + h2 : cx - h2;
-            cy = (o & 2u) ? cy + h2 : cy - h2;
-            if (DIM == 3) cz = (o & 4u) ? cz + h2 : cz - h2;
-            ext = h2;
-            if (l >= lmax) {
-                const int t = l - lmax;
-                const uint64_t dig = (uint64_t)o << (DIM * (W - 1 - t % W));
-                w0 |= t < W ? dig : 0ull;
-                w1 |= t >= W && t < 2 * W ? dig : 0ull;
-                w2 |= t >= 2 * W ? dig : 0ull;
-            }
-        }
-        deep[j] = DeepKey{{w0, w1, w2}};
+        deep[j] = deep_key<DIM>(key, d.spos[src], E, lmax);
     }
     for (uint64_t j = g + 1; j <= r; ++j) {
         const DeepKey kv = deep[j];
@@ -1672,11 +1698,12 @@ __device__ __forceinline__ void minmax_lanes(uint64_t& lo, uint64_t& hi) {
     hi = b > hi ? b : hi;
 }
 
+template <int E>
 __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
                                                   uint32_t* __restrict__ vals, uint64_t base,
                                                   uint32_t cnt, uint8_t* s_raw,
                                                   const uint64_t* __restrict__ quant,
-                                                  uint32_t& heads) {
+                                                  bool& ties) {
     constexpr int kWaves = kBucketThreads / 64;
     uint64_t* s_k = reinterpret_cast<uint64_t*>(s_raw);
     uint32_t* s_v = reinterpret_cast<uint32_t*>(s_raw + kSlots * 8);
@@ -1694,10 +1721,10 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     // the bucket, cnt >= 2: a load inside a divergent branch is waited for at
     // the branch's end)
     const uint64_t qv = quant ? quant[min(t, kCoarse - 1u)] : 0ull;
-    uint64_t key[4];
-    uint32_t val[4];
+    uint64_t key[E];
+    uint32_t val[E];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint64_t i = base + min((uint32_t)e * kBucketThreads + t, cnt - 1u);
         key[e] = keys[i];
         val[e] = vals[i];
@@ -1711,7 +1738,7 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     }
     uint64_t lo = ~0ull, hi = 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         if ((uint32_t)e * kBucketThreads + t < cnt) {
             lo = key[e] < lo ? key[e] : lo;
             hi = key[e] > hi ? key[e] : hi;
@@ -1737,9 +1764,9 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     const uint64_t range = hi - lo;
     const int bits = range ? 64 - __clzll((long long)range) : 0;
     const int sh = bits > kCoarseBits ? bits - kCoarseBits : 0;
-    uint32_t slot[4], rank[4], frac[4];
+    uint32_t slot[E], rank[E], frac[E];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint32_t i = (uint32_t)e * kBucketThreads + t;
         if (quant) {
             // the last quantile <= key (the first if none)
@@ -1771,7 +1798,7 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint32_t i = (uint32_t)e * kBucketThreads + t;
         rank[e] = 0;
         if (i < cnt) {
@@ -1785,7 +1812,8 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     // this thread's slots 4t .. 4t + 3
     const uint32_t w0 = s_pos[2 * t], w1 = s_pos[2 * t + 1];
     const uint32_t c0 = w0 & 0xFFFFu, c1 = w0 >> 16, c2 = w1 & 0xFFFFu, c3 = w1 >> 16;
-    if (__syncthreads_or(max(max(c0, c1), max(c2, c3)) > 64u)) return false;
+    if (uniform_u32((uint32_t)__syncthreads_or(max(max(c0, c1), max(c2, c3)) > 64u)) != 0)
+        return false;
     const uint32_t cs[4] = {c0, c1, c2, c3};
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -1797,12 +1825,13 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     const uint32_t s0 = block_exclusive_scan<kBucketThreads>(c0 + c1 + c2 + c3, s_scan, &all);
     const uint32_t s1 = s0 + c0, s2 = s1 + c1, s3 = s2 + c2;
     // (the scan's barriers ordered the wide-slot count)
-    if (s_wide[0] > kWideSlots) return false;
+    // (told to be uniform: a divergent exit keeps the values of both ways live)
+    if (uniform_u32(s_wide[0]) > kWideSlots) return false;
     s_pos[2 * t] = s0 | (s1 << 16);
     s_pos[2 * t + 1] = s2 | (s3 << 16);
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint32_t i = (uint32_t)e * kBucketThreads + t;
         if (i < cnt) {
             const uint32_t p =
@@ -1815,9 +1844,9 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     // a slot of 2 .. kSlotRun keys: each key's place is its rank among the
     // slot's keys, equal keys keeping their arrival order (a stable sort);
     // the ranks are read first (independent loads), then every key moves
-    uint32_t dst[4];
+    uint32_t dst[E];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint32_t i = (uint32_t)e * kBucketThreads + t;
         dst[e] = ~0u;
         if (i < cnt) {
@@ -1840,7 +1869,7 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
     }
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         if (dst[e] != ~0u) {
             s_k[dst[e]] = key[e];
             s_v[dst[e]] = val[e];
@@ -1861,20 +1890,91 @@ __device__ __forceinline__ bool bucket_sort_slots(uint64_t* __restrict__ keys,
         }
     }
     __syncthreads();
-    // the sorted bucket goes out; bit e of `heads` marks the thread's key e
-    // as the head of a run of equal keys (equal keys share a bucket)
-    uint32_t h = 0;
+    // the sorted bucket goes out; ties: one of the thread's keys heads a run of
+    // equal keys (equal keys share a bucket)
+    bool h = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < E; ++e) {
         const uint32_t i = (uint32_t)e * kBucketThreads + t;
         if (i < cnt) {
             const uint64_t k = s_k[i];
             keys[base + i] = k;
             vals[base + i] = s_v[i];
-            if (i + 1u < cnt && s_k[i + 1u] == k && (i == 0 || s_k[i - 1u] != k)) h |= 1u << e;
+            h |= i + 1u < cnt && s_k[i + 1u] == k;
         }
     }
-    heads = h;
+    ties = h;
+    return true;
+}
+
+// The runs of equal keys of a bucket that the slot sort left in LDS (s_k,
+// s_v), put in (deep key, index) order in vals and deep. Every member finds
+// its own deep key and its rank in its run, all members at once and from LDS:
+// one run's first thread doing all of it (order_tie_run) is a chain of 10 us
+// of global round trips, and one tie in a bucket made the launch that much
+// longer (two clusters of 1M bodies, 21 ties a step: 37 us, 27 now; 64 uneven
+// spheres, 3 ties: 34, 27). More members than the space holds: false, nothing
+// ordered. All threads call.
+constexpr uint32_t kTieSpace = 680;  // members (24 bytes each) in the sort space
+template <int DIM>
+__device__ __forceinline__ bool order_ties_lds(const SegDesc* __restrict__ desc,
+                                               uint32_t* __restrict__ vals,
+                                               DeepKey* __restrict__ deep, uint32_t nseg,
+                                               int segbits, int lmax, uint64_t base, uint32_t cnt,
+                                               const uint64_t* s_k, const uint32_t* s_v,
+                                               uint16_t* s_place, uint32_t* s_n, DeepKey* s_deep) {
+    constexpr uint32_t kNone = 0xFFFFu;
+    // the run of body i: [a, z), z = a when it has none (a slot holds at most
+    // 64 keys)
+    auto run_of = [&](uint32_t i, uint32_t& a, uint32_t& z) {
+        const uint64_t k = s_k[i];
+        a = i;
+        z = i + 1u;
+        while (a > 0 && s_k[a - 1u] == k) --a;
+        while (z < cnt && s_k[z] == k) ++z;
+        if (z - a < 2u) z = a;
+    };
+    if (threadIdx.x == 0) *s_n = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t i = threadIdx.x; i < cnt; i += kBucketThreads) {
+        uint32_t a, z;
+        run_of(i, a, z);
+        const uint64_t key = s_k[i];
+        const uint32_t s = seg_of_key(key, segbits);
+        if (z != a && s < nseg) {
+            const SegDesc& d = desc[s];
+            const uint64_t src = (uint64_t)s_v[i] - d.off;
+            uint32_t p = kNone;
+            if (src < d.n) {
+                const double E = bits_f64(d.st->extent_bits);
+                p = atomicAdd(s_n, 1u);
+                if (p < kTieSpace) s_deep[p] = deep_key<DIM>(key, d.spos[src], E, lmax);
+            } else {
+                atomicOr(&d.st->err, kErrCapacity);
+            }
+            s_place[i] = (uint16_t)p;
+        }
+    }
+    __syncthreads();
+    if (uniform_u32(*s_n) > kTieSpace) return false;
+#pragma unroll 1
+    for (uint32_t i = threadIdx.x; i < cnt; i += kBucketThreads) {
+        uint32_t a, z;
+        run_of(i, a, z);
+        if (z != a && seg_of_key(s_k[i], segbits) < nseg) {
+            // (a member out of its segment, an error: the run stays)
+            uint32_t r = 0, none = 0;
+            for (uint32_t j = a; j < z; ++j) none |= s_place[j] == kNone ? 1u : 0u;
+            if (!none) {
+                const DeepKey mine = s_deep[s_place[i]];
+                for (uint32_t j = a; j < z; ++j)
+                    r += j != i && deep_less<DIM>(s_deep[s_place[j]], s_v[j], mine, s_v[i]) ? 1u : 0u;
+                deep[base + a + r] = mine;
+                vals[base + a + r] = s_v[i];
+            }
+        }
+    }
     return true;
 }
 
@@ -1898,6 +1998,9 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
     static_assert(kSlots * 14 + 16 * kWaves + 4 * kWaves + 12 * kCoarse + 4 * (1 + kWideSlots) <=
                       kSortBytes,
                   "slot sort in the sort space");
+    static_assert(kSlots * 14 + 20 * kWaves + 8 + sizeof(DeepKey) * kTieSpace <= kSortBytes &&
+                      (kSlots * 14 + 20 * kWaves) % 8 == 0 && kTieSpace < 0xFFFF,
+                  "tied bodies in the sort space");
     __shared__ __align__(16) uint8_t s_raw[kSortBytes > kRankBytes ? kSortBytes : kRankBytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t cnt = bcount[blockIdx.x];
@@ -1921,81 +2024,81 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
     if (cnt <= min(cap, (uint32_t)kBucketCap)) {
         uint64_t* s_bk = reinterpret_cast<uint64_t*>(s_raw);
         uint32_t* s_bv = reinterpret_cast<uint32_t*>(s_raw + kBucketCap * 8);
-        uint32_t heads = 0;
-        const bool slots =
-            cnt <= kSlots &&
-            bucket_sort_slots(keys, vals, base, cnt, s_raw,
-                              sc->quantiles ? quant + (uint64_t)blockIdx.x * kQuantiles : nullptr,
-                              heads);
-        if (!slots) {
-            __syncthreads();  // (the slot sort's tables share the space)
+        bool ties = false;
+        const uint64_t* q = sc->quantiles ? quant + (uint64_t)blockIdx.x * kQuantiles : nullptr;
+        bool slots = false;
+        if (cnt <= kSlots / 4) slots = bucket_sort_slots<1>(keys, vals, base, cnt, s_raw, q, ties);
+        else if (cnt <= kSlots / 2)
+            slots = bucket_sort_slots<2>(keys, vals, base, cnt, s_raw, q, ties);
+        else if (cnt <= kSlots) slots = bucket_sort_slots<4>(keys, vals, base, cnt, s_raw, q, ties);
+        __syncthreads();
+        if (slots) {
+            if (uniform_u32((uint32_t)__syncthreads_or(ties)) == 0) return;
+            uint8_t* space = s_raw + kSlots * 14 + 16 * kWaves + 4 * kWaves;
+            if (order_ties_lds<DIM>(desc, vals, deep, nseg, segbits, lmax, base, cnt,
+                                    reinterpret_cast<const uint64_t*>(s_raw),
+                                    reinterpret_cast<const uint32_t*>(s_raw + kSlots * 8),
+                                    reinterpret_cast<uint16_t*>(s_raw + kSlots * 12),
+                                    reinterpret_cast<uint32_t*>(space),
+                                    reinterpret_cast<DeepKey*>(space + 8)))
+                return;
+        } else {
+            // (the slot sort's tables share the space)
             if (cnt <= 2u * kBucketThreads) bucket_sort_regs<2>(keys, vals, base, cnt, s_bk, s_bv);
             else if (cnt <= 4u * kBucketThreads) bucket_sort_regs<4>(keys, vals, base, cnt, s_bk, s_bv);
             else bucket_sort_regs<8>(keys, vals, base, cnt, s_bk, s_bv);
         }
-        __syncthreads();
-        if (slots) {
-            // only the heads the slot sort marked start runs of equal keys
-#pragma unroll 1
-            for (int e = 0; e < 4; ++e)
-                if ((heads >> e) & 1u)
-                    order_tie_run<DIM>(desc, total, keys, vals, deep, nseg, segbits, lmax,
-                                       base + (uint32_t)e * kBucketThreads + (uint32_t)tid);
-        } else {
+    } else {
+        // HBM: stable LSD passes over the range, chunk by chunk in order
+        uint64_t diff = 0;
+        for (uint32_t i = tid; i < cnt; i += kBucketThreads) diff |= keys[base + i] ^ ref;
+        const int hb = block_top_diff_bit(diff, s_or);
+        uint64_t *ka = keys + base, *kb = tkeys + base;
+        uint32_t *va = vals + base, *vb = tvals + base;
+        for (int shift = 0; shift <= hb; shift += 8) {
+            // digit totals of the range, then running starts
+            if (tid < 256) s_run[tid] = 0;
+            __syncthreads();
             for (uint32_t i = tid; i < cnt; i += kBucketThreads)
-                order_tie_run<DIM>(desc, total, keys, vals, deep, nseg, segbits, lmax, base + i);
-        }
-        return;
-    }
-    // HBM: stable LSD passes over the range, chunk by chunk in order
-    uint64_t diff = 0;
-    for (uint32_t i = tid; i < cnt; i += kBucketThreads) diff |= keys[base + i] ^ ref;
-    const int hb = block_top_diff_bit(diff, s_or);
-    uint64_t *ka = keys + base, *kb = tkeys + base;
-    uint32_t *va = vals + base, *vb = tvals + base;
-    for (int shift = 0; shift <= hb; shift += 8) {
-        // digit totals of the range, then running starts
-        if (tid < 256) s_run[tid] = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < cnt; i += kBucketThreads)
-            atomicAdd(&s_run[(uint32_t)((ka[i] >> shift) & 255u)], 1u);
-        __syncthreads();
-        uint32_t total;
-        const uint32_t start = block_exclusive_scan<kBucketThreads>(tid < 256 ? s_run[tid] : 0u,
-                                                                    s_scan, &total);
-        if (tid < 256) s_run[tid] = start;
-        __syncthreads();
-        for (uint32_t c0 = 0; c0 < cnt; c0 += kBucketChunk) {
-            uint64_t key[4];
-            uint32_t val[4], dig[4], pos[4];
+                atomicAdd(&s_run[(uint32_t)((ka[i] >> shift) & 255u)], 1u);
+            __syncthreads();
+            uint32_t total;
+            const uint32_t start = block_exclusive_scan<kBucketThreads>(tid < 256 ? s_run[tid] : 0u,
+                                                                        s_scan, &total);
+            if (tid < 256) s_run[tid] = start;
+            __syncthreads();
+            for (uint32_t c0 = 0; c0 < cnt; c0 += kBucketChunk) {
+                uint64_t key[4];
+                uint32_t val[4], dig[4], pos[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t i = c0 + (uint32_t)wave * 256u + (uint32_t)k * 64u + (uint32_t)lane;
-                const bool valid = i < cnt;
-                key[k] = valid ? ka[i] : 0ull;
-                val[k] = valid ? va[i] : 0u;
-                dig[k] = valid ? (uint32_t)((key[k] >> shift) & 255u) : 256u;
-            }
-            chunk_rank(dig, pos, s_wcnt, s_dstart, s_dcnt, s_scan);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                if (dig[k] < 256u) {
-                    const uint32_t o = s_run[dig[k]] + (pos[k] - s_dstart[dig[k]]);
-                    kb[o] = key[k];
-                    vb[o] = val[k];
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t i = c0 + (uint32_t)wave * 256u + (uint32_t)k * 64u + (uint32_t)lane;
+                    const bool valid = i < cnt;
+                    key[k] = valid ? ka[i] : 0ull;
+                    val[k] = valid ? va[i] : 0u;
+                    dig[k] = valid ? (uint32_t)((key[k] >> shift) & 255u) : 256u;
                 }
+                chunk_rank(dig, pos, s_wcnt, s_dstart, s_dcnt, s_scan);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (dig[k] < 256u) {
+                        const uint32_t o = s_run[dig[k]] + (pos[k] - s_dstart[dig[k]]);
+                        kb[o] = key[k];
+                        vb[o] = val[k];
+                    }
+                }
+                __syncthreads();
+                if (tid < 256) s_run[tid] += s_dcnt[tid];
+                __syncthreads();
             }
-            __syncthreads();
-            if (tid < 256) s_run[tid] += s_dcnt[tid];
-            __syncthreads();
+            uint64_t* tk = ka; ka = kb; kb = tk;
+            uint32_t* tv = va; va = vb; vb = tv;
         }
-        uint64_t* tk = ka; ka = kb; kb = tk;
-        uint32_t* tv = va; va = vb; vb = tv;
-    }
-    if (ka != keys + base) {
-        for (uint32_t i = tid; i < cnt; i += kBucketThreads) {
-            keys[base + i] = ka[i];
-            vals[base + i] = va[i];
+        if (ka != keys + base) {
+            for (uint32_t i = tid; i < cnt; i += kBucketThreads) {
+                keys[base + i] = ka[i];
+                vals[base + i] = va[i];
+            }
         }
     }
     __syncthreads();
@@ -2405,27 +2508,6 @@ __device__ __forceinline__ Sum4 range_sum_row(const double* s_m, const double* s
     return r;
 }
 
-// The reference's descent to a cell (child centres, octree.rs:160-215 /
-// quadtree.rs:161-194):
-// n levels down from a cell of half-width ext and centre c, the half-width
-// halves and the centre moves by it along each axis, up where the key's
-// octant bit is set, else down. w holds the digits to follow inverted and
-// left-aligned (the next digit's DIM bits on top, x lowest), so a digit's
-// inverted bit is the sign of that axis' move; c + (-h) is c - h exactly.
-template <int DIM>
-__device__ __forceinline__ void descend_w(uint64_t w, int n, double& ext, double& cx, double& cy,
-                                          double& cz) {
-    for (int l = 0; l < n; ++l) {
-        const uint32_t top = (uint32_t)(w >> 32);
-        ext = half(ext);
-        const uint64_t hb = f64_bits(ext);
-        const uint32_t lo = (uint32_t)hb, hi = (uint32_t)(hb >> 32);
-        cx += __hiloint2double((int)(hi | ((top << (DIM - 1)) & 0x80000000u)), (int)lo);
-        cy += __hiloint2double((int)(hi | ((top << (DIM - 2)) & 0x80000000u)), (int)lo);
-        if (DIM == 3) cz += __hiloint2double((int)(hi | (top & 0x80000000u)), (int)lo);
-        w <<= DIM;
-    }
-}
 // Levels [from, to) of a body's path: the first key word's digits, then the
 // deep key's (levels past lmax, bodies whose first words tie).
 template <int DIM>

@@ -54,3 +54,32 @@ def test_tiles_around_the_node_list(engine, pairs):
     a = P.Sim(engine, s, kind="astro", theta=0.7, e=0.1, precision="fp64").accel()
     r = np.linalg.norm(a - ref, axis=1) / np.linalg.norm(ref, axis=1)
     assert np.quantile(r, 0.99) <= 1e-11 and r.max() <= 1e-8
+
+
+@pytest.mark.parametrize("pairs,run", [(1, 2), (10, 2), (339, 2), (340, 2), (341, 2), (700, 2),
+                                       (40, 3), (16, 40), (4, 64), (3, 65), (2, 256)])
+def test_tied_first_words(engine, pairs, run):
+    """`pairs` runs of `run` bodies in one cell of level 21 each, beside single
+    ones, in one bucket: up to 680 tied bodies are ordered from LDS, more (and
+    runs past a slot's 64 keys) run by run. First and later passes against the
+    radix sort's, which orders every run by one thread: the same bits."""
+    rng = np.random.default_rng(pairs * 1000 + run)
+    n = pairs * run + 50
+    s = np.zeros(n, P.ENTITY)
+    cells = rng.choice(1 << 18, pairs, replace=False)
+    for k, f in enumerate("xyz"):
+        s[f][:pairs * run] = np.repeat(((cells >> (6 * k)) & 63) / 64.0, run) + 2e-7 \
+            + rng.uniform(0.0, 5e-7, pairs * run)
+        s[f][pairs * run:] = rng.uniform(-1.0, 0.0, 50)
+    s["x"][-1] = -1.0  # the extent: cells of level 21 are 2^-20 wide
+    s["mass"] = rng.uniform(0.5, 1.5, n)
+    kw = dict(kind="astro2", theta=0.7, e=0.1, precision="fp64")
+    radix = P.Engine(0)
+    radix.set_sort(max_buckets=0)
+    other = P.Sim(radix, s, **kw)
+    sim = P.Sim(engine, s, **kw)
+    for _ in range(3):
+        assert sim.accel().tobytes() == other.accel().tobytes()
+    assert sim.stats() == other.stats()
+    sim.close()
+    radix.close()
