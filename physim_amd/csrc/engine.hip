@@ -723,15 +723,20 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
                                                           bp.buckets, e->spl, e->spc, e->bcount,
                                                           e->bfill, e->sc, 1);
         });
+    auto key_tiles = [&](int items) {
+        return (unsigned)((total + items * kKeyThreads - 1) / (items * kKeyThreads));
+    };
     launch(e, cap, "keys", [&] {
-#define PG_KEYS(F)                                                                             \
-    k_keys<DIM, F><<<sort_tiles, kKeyThreads, 0, st>>>(                                        \
+#define PG_KEYS(F, ITEMS)                                                                      \
+    k_keys<DIM, F, ITEMS><<<key_tiles(ITEMS), kKeyThreads, 0, st>>>(                                        \
         desc, e->seg_off, bp.nseg, total, bp.segbits, bp.lmax, e->ext_partial, e->sc,          \
         INTEG ? 1 : 0, bp.buckets ? bp.sort_tag : 0ull, e->keys[0], e->vals[0], e->sort_cnt,   \
         sort_tiles, e->keys[1], bp.buckets, e->bkt, e->bcount, e->quant, e->spl, e->spc)
-        if (!fuse) PG_KEYS(0);
-        else if (!wide) PG_KEYS(1);
-        else PG_KEYS(2);
+        constexpr int kTileItems = kSortTile / kKeyThreads;
+        if (!fuse) PG_KEYS(0, kTileItems);
+        else if (wide) PG_KEYS(2, kTileItems);
+        else if (total <= kFewKeys) PG_KEYS(1, 1);
+        else PG_KEYS(1, 2);
 #undef PG_KEYS
     });
     if (bp.buckets && wide) {
@@ -1161,6 +1166,10 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
         // a batch past max_buckets of bucket_keys grows its buckets up to
         // the slot sort's reach (kSlots keys) before it takes the radix sort
         uint64_t keys_per = e->bucket_keys;
+        if (bp.total <= kFewBodies)
+            keys_per = std::min<uint64_t>(keys_per, kBucketKeysFew);
+        else if (bp.total <= kMoreBodies)
+            keys_per = std::min<uint64_t>(keys_per, kBucketKeysMore);
         if (e->max_buckets && (bp.total + keys_per - 1) / keys_per > e->max_buckets)
             keys_per = std::max<uint64_t>(keys_per, (bp.total + e->max_buckets - 1) / e->max_buckets);
         const uint64_t nb = (bp.total + keys_per - 1) / keys_per;

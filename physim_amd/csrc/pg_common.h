@@ -17,6 +17,14 @@ constexpr int kMaxPasses = 8;      // 8-bit digits over a 64-bit key
 constexpr int kKeyThreads = 512;   // threads of a key-building block (one sort tile)
 constexpr int kBucketKeys = 1664;  // keys per bucket of the sample sort (on average; steady-state
                                    // buckets stay within 2048, the slot sort's reach)
+// The same in small batches, which are far from filling the GPU: shorter
+// buckets are one or two keys a thread, and more blocks (mean 1664: sort of
+// 10,002 bodies 12.1 us, 131,072 14.4, 524,288 16.4; 384: 9.0 and 9.9, but 18 at
+// 524,288, where past kMaxBuckets splitters keys take longer too; 1024: 15.1).
+constexpr int kBucketKeysFew = 384;    // up to kFewBodies bodies
+constexpr int kBucketKeysMore = 1024;  // up to kMoreBodies
+constexpr uint64_t kFewBodies = 1u << 17, kMoreBodies = 1u << 19;
+constexpr uint64_t kFewKeys = 1u << 18;  // up to here a thread builds one key, not two
 constexpr int kBucketCap = 4096;   // largest bucket sorted in LDS (larger ones: in HBM)
 constexpr int kMinBucketKeys = 256;  // smallest mean bucket a tuning may ask for
 constexpr int kBucketThreads = 512;   // threads of a bucket-sorting block (up to 8 keys each)

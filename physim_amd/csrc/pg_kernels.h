@@ -446,14 +446,18 @@ __device__ __forceinline__ uint64_t morton_key(double px, double py, double pz,
 // zero) and the finer quantiles for the slot sort (FUSE 1). FUSE 2 (more than
 // kMaxBuckets buckets) does the work of k_bucket_count_wide: the splitters
 // (spl) and their coarse table (spc) come from k_splitters_wide, run first.
-// One block per radix-sort tile of kSortTile bodies (the batch's segments are
-// concatenated), which also writes the tile's digit counts of the first radix
-// pass (digit-major: cnt[digit * tiles + tile]). The extent
+// One block per tile of ITEMS keys a thread (the batch's segments are
+// concatenated); a radix-sort tile of kSortTile also writes its digit counts of
+// the first pass (digit-major: cnt[digit * tiles + tile]). With FUSE 1 a thread
+// builds one key up to kFewKeys bodies and two past it: a tile is a chain of
+// loads, key digits and a search over the splitters per key, and more blocks
+// hide more of it (four keys, then one or two: 10,002 bodies 11.1 and 8.0 us,
+// 262,144 13.2 and 9.8, 1M 22.8 and 21.6, 1.3M in 64 segments 37 and 31). The extent
 // (transformers.rs:126-131) is the maximum of the segment's chunk partials,
 // reduced by the whole block when the tile lies in one segment; the thread of
 // a segment's first body stores it and opens the segment's step, and block 0
 // resets the batch counters.
-template <int DIM, int FUSE>
+template <int DIM, int FUSE, int ITEMS>
 __global__ __launch_bounds__(kKeyThreads) void k_keys(
     const SegDesc* __restrict__ desc, const uint64_t* __restrict__ seg_off, uint32_t nseg,
     uint64_t total, int segbits, int lmax, const uint64_t* __restrict__ partial,
@@ -470,11 +474,13 @@ __global__ __launch_bounds__(kKeyThreads) void k_keys(
     // bucket counts: of all buckets (FUSE 1), or of a window from s_wb (FUSE 2)
     __shared__ uint32_t s_bh[kMaxBuckets];
     __shared__ uint32_t s_wb;
-    constexpr int kItems = kSortTile / kKeyThreads;
+    constexpr int kItems = ITEMS;
+    static_assert(FUSE || ITEMS * kKeyThreads == kSortTile, "digits are counted per sort tile");
     constexpr int kSplitItems = kMaxBuckets / kKeyThreads;
     static_assert(kMaxBuckets % kKeyThreads == 0, "splitter loads cover the table");
-    const uint64_t g0 = (uint64_t)blockIdx.x * kSortTile;
-    const uint64_t glast = min(g0 + (uint64_t)kSortTile, total) - 1;
+    constexpr uint64_t kTile = (uint64_t)kItems * kKeyThreads;
+    const uint64_t g0 = (uint64_t)blockIdx.x * kTile;
+    const uint64_t glast = min(g0 + kTile, total) - 1;
     const uint32_t sa = seg_of(seg_off, nseg, g0);
     const uint32_t sb = seg_of(seg_off, nseg, glast);
     const bool one = sa == sb;  // block-uniform
@@ -576,7 +582,7 @@ __global__ __launch_bounds__(kKeyThreads) void k_keys(
             const uint64_t g = g0 + (uint64_t)k * kKeyThreads + threadIdx.x;
             uint32_t dig = 256u;
             tk[k] = 0;
-            if (g < total) {
+            if (g <= glast) {
                 const uint32_t s = seg_of(seg_off, nseg, g);
                 const SegDesc& d = desc[s];
                 uint64_t m = 0;
@@ -617,7 +623,7 @@ __global__ __launch_bounds__(kKeyThreads) void k_keys(
 #pragma unroll
         for (int k = 0; k < kItems; ++k) {
             const uint64_t g = g0 + (uint64_t)k * kKeyThreads + threadIdx.x;
-            const bool valid = g < total;
+            const bool valid = g <= glast;
             const uint32_t b = valid ? bk[k] : 0u;
             if (valid) bkt[g] = (uint16_t)b;
             const uint32_t r = b - wb;  // (wraps past the window below it)
