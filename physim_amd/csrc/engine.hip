@@ -92,6 +92,7 @@ struct pg_engine {
     uint32_t bucket_keys = kBucketKeys;  // keys per sample-sort bucket (mean)
     uint32_t walk_run_log2 = 4;          // walk blocks per XCD run: 2^walk_run_log2
     uint64_t ext_valid = 0;  // batch whose extent partials the last step left (0: none)
+    uint32_t ext_zero = 0;   // partials from the first that are known to be zero
     uint64_t sorted_valid = 0;  // batch whose sample-sorted keys keys[1] holds (0: none)
     uint32_t bucket_cap = kBucketCap;    // larger buckets are sorted in HBM
     uint32_t* node_local = nullptr;  // per-body node offset within its tile
@@ -539,6 +540,7 @@ static uint64_t carve_scratch(pg_engine* e, char* b, uint64_t bodies, uint64_t n
     e->cap_segs = segs;
     e->cap_blocks = blocks;
     e->ext_valid = 0;
+    e->ext_zero = 0;
     e->sorted_valid = 0;
     e->last_sim = nullptr;
     e->up_kind = -1;
@@ -1127,6 +1129,37 @@ static int copy_out(pg_engine* e, const void* src, uint64_t bytes, void* out) {
     });
 }
 
+static uint64_t batch_tag(pg_sim* const* sims, uint32_t count) {
+    uint64_t h = 1469598103934665603ull;
+    auto mix = [&](uint64_t v) {
+        h ^= v;
+        h *= 1099511628211ull;
+    };
+    uint64_t total = 0;
+    for (uint32_t i = 0; i < count; ++i) total += sims[i]->n;
+    mix(total);
+    mix(count);
+    for (uint32_t i = 0; i < count; ++i) {
+        mix((uint64_t)(uintptr_t)sims[i]);
+        mix(sims[i]->n);
+    }
+    return h ? h : 1;
+}
+
+// Where a kernel that writes all of s's positions can leave their extent
+// partials for a batch of s alone: in partials known to be zero.
+static ExtentOut extent_out(pg_engine* e, pg_sim* s) {
+    ExtentOut o{nullptr, e->sc ? &e->sc->ext_tag : nullptr, 0};
+    const uint64_t chunks = (s->n + kExtentChunk - 1) / kExtentChunk;
+    e->ext_valid = 0;
+    if (s->p.kind != PG_KIND_DIRECT && e->sc && chunks <= e->ext_zero) {
+        o.partial = e->ext_partial;
+        o.tag = e->ext_valid = batch_tag(&s, 1);
+        e->ext_zero = 0;
+    }
+    return o;
+}
+
 // Core of every device computation: `steps` steps of all sims together
 // (integrate) or one force evaluation into e->acc_out (no integrate). With
 // `wait` false the caller asks for the status and calls finish_batch.
@@ -1286,20 +1319,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
 
     // the batch's identity for the sample sort: its splitters may come from
     // the keys its previous step sorted only when the same batch ran last
-    {
-        uint64_t h = 1469598103934665603ull;
-        auto mix = [&](uint64_t v) {
-            h ^= v;
-            h *= 1099511628211ull;
-        };
-        mix(bp.total);
-        mix(bp.nseg);
-        for (pg_sim* s : sims) {
-            mix((uint64_t)(uintptr_t)s);
-            mix(s->n);
-        }
-        bp.sort_tag = h ? h : 1;
-    }
+    bp.sort_tag = batch_tag(sims.data(), bp.nseg);
     const bool flips = bp.kind != PG_KIND_DIRECT || integrate;
     uint32_t done = 0;
     // An integrating tree step's walk leaves the next step's extent partials:
@@ -1357,6 +1377,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
         if (!integrate) break;
     }
     e->ext_valid = integrate && tree ? bp.sort_tag : 0;
+    e->ext_zero = !integrate && tree ? bp.nchunks : 0;  // (cleared by k_scan_gather)
     e->sorted_valid = warm_needs_sort ? bp.sort_tag : 0;
     HIP_TRY(hipGetLastError());
 
@@ -1498,15 +1519,13 @@ static int upload_async(pg_sim* s, const Entity* state, uint64_t n) {
         PG_TRY(copy_in(e, s->aos, state, n * sizeof(Entity), &src));
         k_unpack<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, e->stream>>>(
             (const uint64_t*)src, src == s->aos ? nullptr : (uint64_t*)s->aos, n, s->pos[0], s->prv[0], s->vx[0], s->vy[0], s->vz[0], s->st,
-            e->sc ? &e->sc->ext_tag : nullptr);
+            extent_out(e, s));
         HIP_TRY(hipGetLastError());
     } else {
         HIP_TRY(hipMemsetAsync(s->st, 0, sizeof(SegState), e->stream));
     }
     s->stage_steps = 0;
     s->steps_known = 0;
-    // new positions: no extent partials are current
-    e->ext_valid = 0;
     s->uploaded = true;
     if (e->last_sim == s) e->last_sim = nullptr;
     return PG_OK;
@@ -1596,7 +1615,8 @@ static int step_stages(pg_engine* e, pg_sim* s, uint32_t steps) {
     for (uint32_t k = 0; k < steps; ++k) {
         if (s->integ == PG_INTEG_EULER) {
             PG_TRY(run_batch(e, &s, 1, 1, false, false));
-            k_euler_update<<<g, kBlock, 0, e->stream>>>(stage_state(s), e->acc_out, s->p.dt);
+            k_euler_update<<<g, kBlock, 0, e->stream>>>(stage_state(s), e->acc_out, s->p.dt,
+                                                        extent_out(e, s));
             HIP_TRY(hipGetLastError());
         } else {
             k_rk4_begin<<<g, kBlock, 0, e->stream>>>(stage_state(s), base);
@@ -1604,15 +1624,18 @@ static int step_stages(pg_engine* e, pg_sim* s, uint32_t steps) {
             for (int st = 0; st < 4; ++st) {
                 PG_TRY(run_batch(e, &s, 1, 1, false, false));
                 k_rk4_stage<<<g, kBlock, 0, e->stream>>>(stage_state(s), e->acc_out, base, ksum,
-                                                         s->p.dt, st);
+                                                         s->p.dt, st, extent_out(e, s));
                 HIP_TRY(hipGetLastError());
             }
         }
-        e->ext_valid = 0;  // the stage kernels moved the bodies
         // one wait a step: where a pass failed on the device, its error bits
         // are sticky and no later stage has changed the state
         PG_TRY(enqueue_status(e, 1));
-        PG_TRY(finish_batch(e));
+        const int rc = finish_batch(e);
+        if (rc != PG_OK) {
+            e->ext_valid = 0;
+            return rc;
+        }
         s->stage_steps += 1;
     }
     return PG_OK;

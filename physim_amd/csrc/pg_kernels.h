@@ -229,6 +229,7 @@ __global__ void k_prep(const SegDesc* __restrict__ desc, uint32_t nseg, StepCoun
     if (t == 0) {
         sc->gen += 1;
         sc->top_levels = 0;
+        sc->ext_tag = 0;  // (the step moves the bodies)
     }
     for (uint32_t s = t; s < nseg; s += stride) open_segment(desc[s].st, 0, integrate);
 }
@@ -280,6 +281,35 @@ __global__ __launch_bounds__(kBlock) void k_extent_partial(const SegDesc* __rest
         if (__ballot(bad) && (threadIdx.x & 63) == 0) atomicOr(&d.st->err, kErrNonFinite);
         m = block_max_u64(m, s_wave);
         if (threadIdx.x == 0) partial[c] = m;
+    }
+}
+
+// The extent partials of new positions, from the kernel that writes them (an
+// upload, an euler or rk4 stage): one segment's, its partials all zero before.
+// NaN/Inf coordinates set the top bit, which k_keys turns into the error that
+// k_extent_partial flags. Saves that kernel's launch and pass: 2 us of the 84
+// that a transform of 1,002 bodies took, 5 of the 108 of an Euler step of 50,003.
+constexpr uint64_t kExtentBad = 1ull << 63;
+struct ExtentOut {
+    uint64_t* partial;  // NULL: none
+    uint64_t* ext_tag;
+    uint64_t tag;
+};
+// Every thread of a block of kBlock calls for its body j (in: j is one).
+__device__ __forceinline__ void extent_of_block(const ExtentOut& o, uint64_t j, bool in, double x,
+                                                double y, double z) {
+    static_assert(kExtentChunk % kBlock == 0, "a block lies in one chunk");
+    __shared__ uint64_t s_wave[kBlock / 64];
+    if (!o.partial) return;
+    uint64_t m = 0;
+    if (in) {
+        m = f64_bits(fmax(fmax(fabs(x), fabs(y)), fabs(z)));
+        if (!isfinite(x) || !isfinite(y) || !isfinite(z)) m |= kExtentBad;
+    }
+    m = block_max_u64(m, s_wave);
+    if (threadIdx.x == 0) {
+        atomicMax((unsigned long long*)&o.partial[j / kExtentChunk], (unsigned long long)m);
+        if (j == 0) *o.ext_tag = o.tag;
     }
 }
 
@@ -554,6 +584,9 @@ __global__ __launch_bounds__(kKeyThreads) void k_keys(
             mblock = b > mblock ? b : mblock;
         }
         mblock = block_max_u64<kKeyThreads>(mblock, s_wave);
+        if (g0 == d.off && threadIdx.x == 0 && (mblock & kExtentBad))
+            atomicOr(&d.st->err, kErrNonFinite);
+        mblock &= ~kExtentBad;
     } else {
         __syncthreads();
     }
@@ -590,6 +623,8 @@ __global__ __launch_bounds__(kKeyThreads) void k_keys(
                     const uint64_t b = partial[d.chunk0 + c];
                     m = b > m ? b : m;
                 }
+                if (g == d.off && (m & kExtentBad)) atomicOr(&d.st->err, kErrNonFinite);
+                m &= ~kExtentBad;
                 if (g == d.off) open_segment(d.st, m, integrate);
                 const double4 p = d.spos[g - d.off];
                 uint64_t key = morton_key<DIM>(p.x, p.y, p.z, m, lmax);
@@ -4143,8 +4178,8 @@ __global__ __launch_bounds__(kBlock) void k_status(const SegDesc* __restrict__ d
 }
 
 // AoS <-> SoA at the host boundary. An upload also starts the simulation's
-// step state afresh, and no extent partials are current then (ext_tag; may be
-// NULL). A block takes its records in through LDS, word by word in order (a
+// step state afresh and leaves its extent partials where they can be (ext;
+// ext_tag may be NULL). A block takes its records in through LDS, word by word in order (a
 // thread reading its own 80-byte record asks for a line per lane and word), so
 // that `src` may be pinned host memory: a small state needs no copy of its own
 // (64 KB: 22 us against 44 for the runtime's pageable copy); it is kept in
@@ -4154,7 +4189,7 @@ static_assert(sizeof(Entity) % 8 == 0, "records of whole 8-byte words");
 __global__ __launch_bounds__(kBlock) void k_unpack(
     const uint64_t* __restrict__ src, uint64_t* __restrict__ aos, uint64_t n,
     double4* __restrict__ pos, double4* __restrict__ prv, double* vx, double* vy, double* vz,
-    SegState* __restrict__ st, uint64_t* __restrict__ ext_tag) {
+    SegState* __restrict__ st, ExtentOut ext) {
     __shared__ uint64_t rec[kBlock * kEntityWords];
     const uint64_t base = (uint64_t)blockIdx.x * kBlock, i = base + threadIdx.x;
     const uint32_t words = (uint32_t)min((uint64_t)kBlock, n - base) * kEntityWords;
@@ -4171,11 +4206,13 @@ __global__ __launch_bounds__(kBlock) void k_unpack(
     }
     if (i == 0) {
         *st = SegState{};
-        if (ext_tag) *ext_tag = 0;
+        if (ext.ext_tag && !ext.partial) *ext.ext_tag = 0;
     }
     __syncthreads();
+    Entity e{};
+    if (i < n) e = *(const Entity*)(rec + threadIdx.x * kEntityWords);
+    extent_of_block(ext, i, i < n, e.x, e.y, e.z);
     if (i >= n) return;
-    const Entity e = *(const Entity*)(rec + threadIdx.x * kEntityWords);
     pos[i] = make_double4(e.x, e.y, e.z, e.mass);
     prv[i] = make_double4(e.x, e.y, e.z, make_tag((uint32_t)i, e.fixed != 0));
     vx[i] = e.vx; vy[i] = e.vy; vz[i] = e.vz;
@@ -4250,19 +4287,26 @@ __device__ __forceinline__ bool stage_failed(const StageState& s) {
 
 // euler.rs:26-45: x' = x + v dt + 0.5 a dt^2 (dt.powi(2) = dt * dt),
 // v' = v + a dt, every body (fixed ones have a = 0 and keep moving).
-__global__ void k_euler_update(StageState st, const double* __restrict__ acc, double dt) {
-    const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= st.n || stage_failed(st)) return;
-    const double* a = acc + 3 * (uint64_t)tag_id(st.prv[j].w);
-    const double dt2 = dt * dt;
-    const double4 p = st.pos[j];
-    const double x = p.x, y = p.y, z = p.z;
-    const double vx = st.vx[j], vy = st.vy[j], vz = st.vz[j];
-    st.pos[j] = make_double4(x + vx * dt + 0.5 * a[0] * dt2, y + vy * dt + 0.5 * a[1] * dt2,
-                             z + vz * dt + 0.5 * a[2] * dt2, p.w);
-    st.vx[j] = vx + a[0] * dt;
-    st.vy[j] = vy + a[1] * dt;
-    st.vz[j] = vz + a[2] * dt;
+__global__ __launch_bounds__(kBlock) void k_euler_update(StageState st,
+                                                         const double* __restrict__ acc, double dt,
+                                                         ExtentOut ext) {
+    const uint64_t j = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    const bool in = j < st.n;
+    const double4 p = st.pos[in ? j : 0];
+    double4 q = p;
+    if (in && !stage_failed(st)) {
+        const double* a = acc + 3 * (uint64_t)tag_id(st.prv[j].w);
+        const double dt2 = dt * dt;
+        const double x = p.x, y = p.y, z = p.z;
+        const double vx = st.vx[j], vy = st.vy[j], vz = st.vz[j];
+        q = make_double4(x + vx * dt + 0.5 * a[0] * dt2, y + vy * dt + 0.5 * a[1] * dt2,
+                         z + vz * dt + 0.5 * a[2] * dt2, p.w);
+        st.pos[j] = q;
+        st.vx[j] = vx + a[0] * dt;
+        st.vy[j] = vy + a[1] * dt;
+        st.vz[j] = vz + a[2] * dt;
+    }
+    extent_of_block(ext, j, in, q.x, q.y, q.z);
 }
 
 // The base state (x, v) of an rk4 step, saved in upload order.
@@ -4282,37 +4326,42 @@ __global__ void k_rk4_begin(StageState st, double* __restrict__ base) {
 // :55-66, :89-100, :123-134, every body, fixed ones included), or after k4
 // the result base + sum / 6.0, a fixed body keeping its position with zero
 // velocity (:168-174).
-__global__ void k_rk4_stage(StageState st, const double* __restrict__ acc,
-                            const double* __restrict__ base, double* __restrict__ ksum, double dt,
-                            int stage) {
-    const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= st.n || stage_failed(st)) return;
-    const double4 pr = st.prv[j];
-    const uint64_t u = tag_id(pr.w);
-    const double* a = acc + 3 * u;
-    const double* b = base + 6 * u;
-    double* ks = ksum + 6 * u;
-    const double k[6] = {dt * st.vx[j], dt * st.vy[j], dt * st.vz[j],
-                         dt * a[0], dt * a[1], dt * a[2]};
-    double sum[6];
-    for (int c = 0; c < 6; ++c) {
-        if (stage == 0) sum[c] = k[c];
-        else if (stage == 3) sum[c] = ks[c] + k[c];
-        else sum[c] = ks[c] + 2.0 * k[c];
-        ks[c] = sum[c];
+__global__ __launch_bounds__(kBlock) void k_rk4_stage(StageState st, const double* __restrict__ acc,
+                                                      const double* __restrict__ base,
+                                                      double* __restrict__ ksum, double dt,
+                                                      int stage, ExtentOut ext) {
+    const uint64_t j = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    const bool in = j < st.n;
+    const double4 p = st.pos[in ? j : 0];
+    double o[6] = {p.x, p.y, p.z, 0.0, 0.0, 0.0};
+    if (in && !stage_failed(st)) {
+        const double4 pr = st.prv[j];
+        const uint64_t u = tag_id(pr.w);
+        const double* a = acc + 3 * u;
+        const double* b = base + 6 * u;
+        double* ks = ksum + 6 * u;
+        const double k[6] = {dt * st.vx[j], dt * st.vy[j], dt * st.vz[j],
+                             dt * a[0], dt * a[1], dt * a[2]};
+        double sum[6];
+        for (int c = 0; c < 6; ++c) {
+            if (stage == 0) sum[c] = k[c];
+            else if (stage == 3) sum[c] = ks[c] + k[c];
+            else sum[c] = ks[c] + 2.0 * k[c];
+            ks[c] = sum[c];
+        }
+        if (stage < 3) {
+            const double w = stage < 2 ? 0.5 : 1.0;
+            for (int c = 0; c < 6; ++c) o[c] = b[c] + w * k[c];
+        } else if (!tag_fixed(pr.w)) {
+            for (int c = 0; c < 6; ++c) o[c] = b[c] + sum[c] / 6.0;
+        } else {
+            for (int c = 0; c < 3; ++c) o[c] = b[c];
+            for (int c = 3; c < 6; ++c) o[c] = 0.0;
+        }
+        st.pos[j] = make_double4(o[0], o[1], o[2], p.w);
+        st.vx[j] = o[3]; st.vy[j] = o[4]; st.vz[j] = o[5];
     }
-    double o[6];
-    if (stage < 3) {
-        const double w = stage < 2 ? 0.5 : 1.0;
-        for (int c = 0; c < 6; ++c) o[c] = b[c] + w * k[c];
-    } else if (!tag_fixed(pr.w)) {
-        for (int c = 0; c < 6; ++c) o[c] = b[c] + sum[c] / 6.0;
-    } else {
-        for (int c = 0; c < 3; ++c) o[c] = b[c];
-        for (int c = 3; c < 6; ++c) o[c] = 0.0;
-    }
-    st.pos[j] = make_double4(o[0], o[1], o[2], st.pos[j].w);
-    st.vx[j] = o[3]; st.vy[j] = o[4]; st.vz[j] = o[5];
+    extent_of_block(ext, j, in, o[0], o[1], o[2]);
 }
 
 // v = (x - x_prev) / dt (the Stormer velocity, verlet.rs:68-70) written into

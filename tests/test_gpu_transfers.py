@@ -86,3 +86,48 @@ def test_failed_pass_leaves_the_state(engine, integrator):
         assert ei.value.code == 7
         assert sim.download().tobytes() == s.tobytes()
     sim.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 4095, 4097, 20000])
+@pytest.mark.parametrize("kind", ["astro2", "astro"])
+def test_extent_of_uploads_and_stages(engine, kind, n):
+    """The extent left by an upload after a force-only pass, and by each euler
+    and rk4 stage, against passes of a fresh engine, which reduce it from the
+    positions: states that grow and shrink, the largest coordinate in any block
+    and on any axis, non-finite ones. Also through a change to the direct sum
+    and back, whose steps leave no extent."""
+    rng = np.random.default_rng(n)
+    base = np.zeros(n, P.ENTITY)
+    for f in ("x", "y", "z", "vx", "vy", "vz"):
+        base[f] = rng.uniform(-1.0, 1.0, n)
+    base["mass"] = 1.0 / n
+    kw = dict(kind=kind, theta=0.7, e=0.1)
+    fresh = P.Engine(0)
+    for k in range(6):
+        s = base.copy()
+        s["xyz"[k % 3]][rng.integers(n)] = (-1.0) ** k * 10.0 ** (2 - k)
+        a = engine.transform(s, **kw)
+        ref = P.Sim(fresh, s, **kw)
+        assert a.view(np.float64).reshape(-1, 3).tobytes() == ref.accel().tobytes()
+        ref.close()
+        bad = s.copy()
+        bad["xyz"[k % 3]][rng.integers(n)] = (np.inf, -np.inf, np.nan)[k // 2]
+        with pytest.raises(P.PgError) as ei:
+            engine.transform(bad, **kw)
+        assert ei.value.code == 7
+    for integrator in ("euler", "rk4"):
+        sim = P.Sim(engine, base, dt=0.1, **kw)
+        sim.set_integrator(integrator)
+        for _ in range(3):
+            sim.step(1)
+            now = P.Sim(fresh, sim.download(), **kw)
+            assert sim.accel().tobytes() == now.accel().tobytes()
+            now.close()
+        sim.set_params(kind="simple_astro", theta=0.7, e=0.1, dt=0.5)
+        sim.step(2)
+        sim.set_params(dt=0.1, **kw)
+        now = P.Sim(fresh, sim.download(), **kw)
+        assert sim.accel().tobytes() == now.accel().tobytes()
+        now.close()
+        sim.close()
+    fresh.close()
