@@ -698,6 +698,21 @@ static inline unsigned grid_for(uint64_t n, unsigned cap) {
     return (unsigned)std::min<uint64_t>(g, cap);
 }
 
+// How many lanes of a wave walk a body, as a power of two. A wave's time is
+// the items of all its bodies, and a small batch leaves the chip short of
+// waves (1,024 SIMDs): fewer bodies to a wave are more and shorter walks, up
+// to 2,048 waves, or 3,072 where 16 or 32 lanes are used in mixed precision.
+// Past that the idle lanes' issue slots are missed. Steps at 64 lanes and as
+// chosen here, theta 0.5, uniform and clustered bodies, us: 1,000: 120, 158 and
+// 80, 123; 10,000: 187, 257 and 119, 191; 30,000: 224, 302 and 158, 237;
+// 65,536: 226, 331 and 200, 300 (32 lanes at 131,072: 238 and 372 against 259
+// and 366; 16 at 65,536: 188 and 312); theta 1.5: no difference.
+static inline uint32_t walk_lanes_log2(uint64_t total, bool fp64) {
+    for (uint32_t l = 2; l < 6; ++l)
+        if (total <= (fp64 || l < 4 ? 2048ull : 3072ull) << l) return l;
+    return 6;
+}
+
 // `extent`: the extent partials may be stale (the last step did not leave
 // them), so the extent pass runs. `fused`: keys[1] holds this batch's
 // previous sample-sorted keys, so k_keys takes the splitters from them and
@@ -845,11 +860,14 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
                 desc, e->seg_off, bp.nseg, e->tile_start, e->hot, e->top_last, e->top_slot,
                 e->out_part, e->in_part, e->tot_part, e->sc);
         });
+    const uint32_t lanes = walk_lanes_log2(total, FP64);
+    const uint32_t per_block = (kBlock / 64) << lanes;
+    const unsigned walk_blocks = (unsigned)((total + per_block - 1) / per_block);
     launch(e, cap, "walk", [&] {
 #define PG_WALK(NEAR, COUNT)                                                                   \
-    k_walk<DIM, FP64, INTEG, NEAR, COUNT><<<grid_for(total, 1u << 30), kBlock, 0, st>>>(       \
+    k_walk<DIM, FP64, INTEG, NEAR, COUNT><<<walk_blocks, kBlock, 0, st>>>(                    \
         desc, total, skeys, bp.segbits, e->first_node, e->hot, e->cap_nodes, bp.nseg,         \
-        e->acc_out, e->ext_partial, e->sc, bp.sort_tag, e->leaf_lv, e->walk_run_log2,          \
+        e->acc_out, e->ext_partial, e->sc, bp.sort_tag, e->leaf_lv, e->walk_run_log2, lanes,   \
         e->leafpos, e->node_span, svals)
         // (walks without the near-field test or the interaction counters
         // where no segment asks for them hold fewer registers)

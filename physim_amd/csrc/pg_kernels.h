@@ -3487,8 +3487,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     int segbits, const uint32_t* __restrict__ first_node, const NodeHot* __restrict__ hot,
     uint64_t cap, uint32_t nseg, double* __restrict__ acc_out, uint64_t* __restrict__ ext_partial,
     StepCounters* __restrict__ sc, uint64_t tag, const uint8_t* __restrict__ leaf_lv,
-    uint32_t run_log2, const double4* __restrict__ leafpos, const uint2* __restrict__ node_span,
-    const uint32_t* __restrict__ svals) {
+    uint32_t run_log2, uint32_t lanes_log2, const double4* __restrict__ leafpos,
+    const uint2* __restrict__ node_span, const uint32_t* __restrict__ svals) {
     // per wave: the lanes' lists (item numbers within the chunk) and the
     // chunk's sources, all (x, y) then all (z, mass): FP32 mass in mixed
     // precision
@@ -3506,8 +3506,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         const uint32_t x = blockIdx.x & 7u, k = blockIdx.x >> 3;
         blk = (k >> run_log2) * group + (x << run_log2) + (k & ((1u << run_log2) - 1u));
     }
-    const uint64_t g = (uint64_t)blk * blockDim.x + threadIdx.x;
+    // a wave's first 2^lanes_log2 lanes walk (a small batch: more waves, each
+    // with fewer bodies' items; see walk_lanes_log2); the others only fetch
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t lanes = 1u << lanes_log2;
+    const uint64_t g =
+        ((uint64_t)(blk * (kBlock / 64) + wv) << lanes_log2) + (lane & (lanes - 1u));
     // Every load that needs no other goes out at once, at indices clamped into
     // range (a load behind a divergent branch is waited for at the branch's
     // end); a batch of one segment needs no key to name it, and a wave in one
@@ -3536,7 +3540,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     // the body's index in the previous order (k_scan_gather flags one
     // outside its segment; such a body is not stepped)
     const uint64_t j = g - off, src = (uint64_t)v - off;
-    valid = valid && src < n;
+    valid = valid && src < n && lane < lanes;
     const double4 pr = gload(sprv + (valid ? src : 0));  // previous position and tag
     const double x = p.x, y = p.y, z = p.z, m = p.w;
     const bool fixed = !valid || tag_fixed(pr.w);

@@ -36,6 +36,25 @@ def test_alone_equals_beside_a_large_one(engine, filler, kind, model, n):
         x.close()
 
 
+@pytest.mark.parametrize("precision,near", [("fp64", 0.0), ("fp64", 1.5), ("mixed", 1.5)])
+@pytest.mark.parametrize("n", [5, 1023, 8192, 8193, 16385, 32768, 32769, 49152, 49153, 98304])
+def test_fewer_walking_lanes(engine, filler, precision, near, n):
+    """Waves of 4, 8, 16 and 32 walking lanes (alone) against 64 (beside the
+    filler), at their lines in both precisions and with a near field."""
+    s = P.gen_plummer_virial(n, seed=n, mass=1.0, a=0.1)
+    kw = dict(kind="astro2", theta=0.6, e=0.01, dt=1e-4, precision=precision)
+    alone, beside, big = (P.Sim(engine, x, **kw) for x in (s, s, filler))
+    for x in (alone, beside, big):
+        x.set_near_field(near)
+        x.set_counting(True)
+    alone.step(3)
+    engine.batch_step([beside, big], 3)
+    assert alone.download().tobytes() == beside.download().tobytes()
+    assert alone.interaction_counts().tobytes() == beside.interaction_counts().tobytes()
+    for x in (alone, beside, big):
+        x.close()
+
+
 @pytest.mark.parametrize("pairs", [0, 20, 30, 36, 42, 60])
 def test_tiles_around_the_node_list(engine, pairs):
     """One node tile of a quadtree whose internal nodes go from 0.7 to 1.2 per
