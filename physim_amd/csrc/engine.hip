@@ -734,6 +734,8 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
     // previous step's sorted keys give them (fused), else by k_bucket_count_wide
     const bool wide = bp.buckets > e->lds_buckets;
     const bool fuse = fused && bp.buckets;
+    // the sort's blocks collect their keys themselves
+    const bool gather = bp.buckets && total <= (uint64_t)kGatherKeys && bp.buckets <= 64;
     if (fuse && wide)
         launch(e, cap, "splitters", [&] {
             k_splitters_wide<<<1, kSplitThreads, 0, st>>>(e->keys[1], e->keys[0], total,
@@ -790,7 +792,7 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
                                                                     e->quant, e->sc);
             });
         }
-        launch(e, cap, "bucket_scatter", [&] {
+        if (!gather) launch(e, cap, "bucket_scatter", [&] {
             k_bucket_scatter<<<sort_tiles, kSortThreads, 0, st>>>(
                 e->keys[0], e->vals[0], e->bkt, total, e->bcount, e->bfill, e->bbase, nb,
                 e->keys[1], e->vals[1]);
@@ -799,9 +801,14 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
     if (bp.buckets) {
         const uint32_t nb = bp.buckets;
         launch(e, cap, "bucket_sort", [&] {
-            k_bucket_sort<DIM><<<nb, kBucketThreads, 0, st>>>(
-                e->keys[1], e->vals[1], e->keys[0], e->vals[0], e->bcount, e->bfill, e->bbase,
-                e->bucket_cap, desc, total, e->deep, bp.nseg, bp.segbits, bp.lmax, e->quant, e->sc);
+#define PG_SORT(GATHER)                                                                        \
+    k_bucket_sort<DIM, GATHER><<<nb, kBucketThreads, 0, st>>>(                                 \
+        e->keys[1], e->vals[1], e->keys[0], e->vals[0], e->bcount, e->bfill, e->bbase,        \
+        e->bucket_cap, desc, total, e->deep, bp.nseg, bp.segbits, bp.lmax, e->quant, e->sc,   \
+        e->bkt)
+            if (gather) PG_SORT(true);
+            else PG_SORT(false);
+#undef PG_SORT
         });
     } else {
         for (int p = 0; p < bp.passes; ++p) {
@@ -833,7 +840,8 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
     launch(e, cap, "scan_gather", [&] {
         k_scan_gather<DIM><<<tiles, kBlock, 0, st>>>(
             desc, e->tile_start, e->ext_partial, bp.nchunks, skeys, svals, bp.nseg, bp.segbits, bp.lmax, e->node_local,
-            e->tile_tot, e->lo_level, e->lvl_first, e->deep, e->err_global, e->leaf_lv, e->leafpos);
+            e->tile_tot, e->lo_level, e->lvl_first, e->deep, e->err_global, e->leaf_lv, e->leafpos, e->bcount,
+            gather ? bp.buckets : 0u);
     });
     const bool few = tiles <= (unsigned)kFewTiles;
     if (!few)

@@ -25,6 +25,7 @@ constexpr int kBucketKeysFew = 384;    // up to kFewBodies bodies
 constexpr int kBucketKeysMore = 1024;  // up to kMoreBodies
 constexpr uint64_t kFewBodies = 1u << 17, kMoreBodies = 1u << 19;
 constexpr uint64_t kFewKeys = 1u << 18;  // up to here a thread builds one key, not two
+constexpr int kGatherKeys = 16384;  // batches whose sort blocks collect their own keys (no scatter)
 constexpr int kBucketCap = 4096;   // largest bucket sorted in LDS (larger ones: in HBM)
 constexpr int kMinBucketKeys = 256;  // smallest mean bucket a tuning may ask for
 constexpr int kBucketThreads = 512;   // threads of a bucket-sorting block (up to 8 keys each)

@@ -102,3 +102,28 @@ def test_tied_first_words(engine, pairs, run):
     assert sim.stats() == other.stats()
     sim.close()
     radix.close()
+
+
+@pytest.mark.parametrize("n", [700, 1900, 3000, 9000, 16384, 16385])
+def test_keys_far_from_the_last_splitters(engine, n):
+    """A state whose keys all fall in one or two of the buckets that the
+    previous state's keys made (up to 2,048 keys listed, more written out for
+    the other sorts), against a fresh engine."""
+    rng = np.random.default_rng(n)
+    s = np.zeros(n, P.ENTITY)
+    for f in "xyz":
+        s[f] = rng.uniform(-1.0, 1.0, n)
+    s["mass"] = 1.0 / n
+    kw = dict(kind="astro2", theta=0.7, e=0.1)
+    sim = P.Sim(engine, s, **kw)
+    sim.accel()
+    for f in "xyz":
+        s[f][1:] = 0.9 + s[f][1:] * 1e-3
+    s["x"][0] = -1.0
+    sim.upload(s)
+    fresh = P.Engine(0)
+    ref = P.Sim(fresh, s, **kw)
+    for _ in range(2):
+        assert sim.accel().tobytes() == ref.accel().tobytes()
+    sim.close()
+    fresh.close()
