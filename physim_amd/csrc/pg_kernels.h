@@ -472,8 +472,8 @@ __device__ __forceinline__ uint64_t morton_key(double px, double py, double pz,
 // first pass. With FUSE (the sample sort, the batch's previous sorted keys
 // in `prev`) it does the work of k_splitters and k_bucket_count instead: the
 // same splitters (prev at the quantile positions), each key's bucket, the
-// bucket sizes (one atomic per tile and bucket; the bucket sort leaves them
-// zero) and the finer quantiles for the slot sort (FUSE 1). FUSE 2 (more than
+// bucket sizes (one atomic per tile and bucket; the bucket sort, or the
+// gather after it, leaves them zero) and the finer quantiles for the slot sort (FUSE 1). FUSE 2 (more than
 // kMaxBuckets buckets) does the work of k_bucket_count_wide: the splitters
 // (spl) and their coarse table (spc) come from k_splitters_wide, run first.
 // One block per tile of ITEMS keys a thread (the batch's segments are
@@ -2724,8 +2724,8 @@ __device__ __forceinline__ uint4 pack_skip(double a, uint32_t skip, uint32_t lev
 //
 // With FEW (at most kFewTiles tiles) the block does k_tree_scan's work for
 // itself: the tiles' bases from their totals (one wave), the suffix minimum of
-// the tiles after its own from their rows of lvl_first. A launch less, 4 us of
-// the 67 that a step of 10,002 bodies takes, for up to eight loads a thread
+// the tiles after its own from their rows of lvl_first. A launch less, 3 us of
+// the 67 that a step of 10,002 bodies took, for up to eight loads a thread
 // beside the staging's.
 template <int DIM, bool FEW>
 __global__ __launch_bounds__(kNodeThreads) __attribute__((amdgpu_waves_per_eu(6))) void k_nodes(
@@ -3706,7 +3706,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         // first body), else the leaf of body b. After node k the next item is
         // (b, k + 1) when some lane opened it, else (the body after its
         // range, its skip). k is at most the last internal node of the batch
-        // plus one, whose span (k_tree_scan) starts at no body. Each step
+        // plus one, whose span (k_tree_scan, k_nodes) starts at no body. Each step
         // raises b, or k at the same b, so the walk ends.
         WalkState w;
         w.b = lanes_where(walker) ? b0 : bend;
