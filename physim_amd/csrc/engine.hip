@@ -151,6 +151,7 @@ struct pg_engine {
     // pinned host memory: a call's tables on their way to the device and its
     // status on the way back (grown with the batch, freed with the engine),
     // and two halves through which states go up and results come back
+    char* block = nullptr;  // the first of it (one allocation); then apart as they grow
     char* pin = nullptr;
     uint64_t pin_bytes = 0;
     char* ret = nullptr;
@@ -293,8 +294,9 @@ extern "C" void pg_engine_destroy(pg_engine* e) {
         (void)hipEventDestroy(ev.second.b);
     }
     (void)hipStreamDestroy(e->stream);
-    if (e->pin) (void)hipHostFree(e->pin);
-    if (e->ret) (void)hipHostFree(e->ret);
+    if (e->pin && e->pin != e->block) (void)hipHostFree(e->pin);
+    if (e->ret && e->ret != e->block + kPinBytes) (void)hipHostFree(e->ret);
+    if (e->block) (void)hipHostFree(e->block);
     for (hipEvent_t ev : e->ret_ev)
         if (ev) (void)hipEventDestroy(ev);
     delete e;
@@ -969,16 +971,34 @@ static int err_text(uint32_t bits) {
     }
 }
 
+// The engine's first pinned memory, at its first use: room for tables and
+// status, then two halves of kSmallCopy.
+static int ensure_block(pg_engine* e) {
+    if (e->block) return PG_OK;
+    for (hipEvent_t& ev : e->ret_ev)
+        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    char* p = nullptr;
+    if (hipHostMalloc((void**)&p, kPinBytes + 2 * kSmallCopy, hipHostMallocDefault) != hipSuccess)
+        return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)",
+                            (unsigned long long)(kPinBytes + 2 * kSmallCopy));
+    e->block = e->pin = p;
+    e->pin_bytes = kPinBytes;
+    e->ret = p + kPinBytes;
+    e->ret_half = kSmallCopy;
+    return PG_OK;
+}
+
 // Pinned memory of at least `bytes`; what it held before is not kept.
 static int ensure_pinned(pg_engine* e, uint64_t bytes) {
+    PG_TRY(ensure_block(e));
     if (bytes <= e->pin_bytes) return PG_OK;
-    uint64_t want = std::max(e->pin_bytes, kPinBytes);
+    uint64_t want = e->pin_bytes;
     while (want < bytes) want *= 2;
-    if (e->pin) HIP_TRY(hipStreamSynchronize(e->stream));
+    HIP_TRY(hipStreamSynchronize(e->stream));
     char* p = nullptr;
     if (hipHostMalloc((void**)&p, want, hipHostMallocDefault) != hipSuccess)
         return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)", (unsigned long long)want);
-    if (e->pin) (void)hipHostFree(e->pin);
+    if (e->pin != e->block) (void)hipHostFree(e->pin);
     e->pin = p;
     e->pin_bytes = want;
     return PG_OK;
@@ -1082,17 +1102,15 @@ static int finish_batch(pg_engine* e) {
 
 // The halves, large enough for `bytes` at a time or of kReturnBytes.
 static int ensure_halves(pg_engine* e, uint64_t bytes) {
-    const uint64_t half = bytes <= kSmallCopy ? kSmallCopy : kReturnBytes;
-    if (e->ret_half >= half) return PG_OK;
-    for (hipEvent_t& ev : e->ret_ev)
-        if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    PG_TRY(ensure_block(e));
+    if (bytes <= kSmallCopy || e->ret_half == kReturnBytes) return PG_OK;
     HIP_TRY(hipStreamSynchronize(e->stream));
     char* p = nullptr;
-    if (hipHostMalloc((void**)&p, 2 * half, hipHostMallocDefault) != hipSuccess)
-        return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)", (unsigned long long)(2 * half));
-    if (e->ret) (void)hipHostFree(e->ret);
-    e->ret = p;
-    e->ret_half = half;
+    if (hipHostMalloc((void**)&p, 2 * kReturnBytes, hipHostMallocDefault) != hipSuccess)
+        return pg_set_error(PG_ERR_NOMEM, "hipHostMalloc(%llu)",
+                            (unsigned long long)(2 * kReturnBytes));
+    e->ret = p;  // (the small ones stay in the block)
+    e->ret_half = kReturnBytes;
     return PG_OK;
 }
 
