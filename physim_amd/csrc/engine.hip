@@ -5,6 +5,7 @@
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <cassert>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -802,12 +803,18 @@ static void enqueue_tree_step(pg_engine* e, const BatchPlan& bp, int q, bool cap
     }
     if (bp.buckets) {
         const uint32_t nb = bp.buckets;
+        // where the blocks collect their keys, all of them read keys[0]: what
+        // one block writes lies elsewhere (the position records are written
+        // after the sort)
+        uint64_t* spare = gather ? reinterpret_cast<uint64_t*>(e->leafpos) : e->keys[0];
+        static_assert(sizeof(*e->leafpos) >= sizeof(uint64_t), "a key per position record");
+        assert(!gather || (spare != e->keys[0] && spare != e->keys[1]));
         launch(e, cap, "bucket_sort", [&] {
 #define PG_SORT(GATHER)                                                                        \
     k_bucket_sort<DIM, GATHER><<<nb, kBucketThreads, 0, st>>>(                                 \
-        e->keys[1], e->vals[1], e->keys[0], e->vals[0], e->bcount, e->bfill, e->bbase,        \
+        e->keys[1], e->vals[1], spare, e->vals[0], e->bcount, e->bfill, e->bbase,             \
         e->bucket_cap, desc, total, e->deep, bp.nseg, bp.segbits, bp.lmax, e->quant, e->sc,   \
-        e->bkt)
+        e->bkt, GATHER ? e->keys[0] : nullptr)
             if (gather) PG_SORT(true);
             else PG_SORT(false);
 #undef PG_SORT

@@ -2037,7 +2037,11 @@ __device__ __forceinline__ bool order_ties_lds(const SegDesc* __restrict__ desc,
 // 16-byte loads a thread) and lists its own in LDS, or writes them out where
 // they are more than the slot sort takes. A launch less than a scatter of their
 // own: a step of 10,000 bodies takes 53.6 us instead of 57.9, a transform of
-// 1,002 70 instead of 82.
+// 1,002 70 instead of 82. Every block then reads the unsorted keys (`from`) at
+// any index and at any time of the launch, so no block writes them: `tkeys` is
+// memory that nothing else in the launch reads or writes, and every other array
+// a block writes it reads and writes in its own bucket's range only. (Without
+// GATHER the scatter has read the unsorted keys, and tkeys may be their array.)
 template <int DIM, bool GATHER>
 __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(GATHER ? 4 : 6))) void k_bucket_sort(
     uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, uint64_t* __restrict__ tkeys,
@@ -2045,7 +2049,7 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
     const uint32_t* __restrict__ bbase, uint32_t cap, const SegDesc* __restrict__ desc,
     uint64_t total, DeepKey* __restrict__ deep, uint32_t nseg, int segbits, int lmax,
     const uint64_t* __restrict__ quant, const StepCounters* __restrict__ sc,
-    const uint16_t* __restrict__ bkt) {
+    const uint16_t* __restrict__ bkt, const uint64_t* __restrict__ from) {
     constexpr int kWaves = kBucketThreads / 64;
     static_assert(kBucketCap == 8 * kBucketThreads, "up to eight keys per thread");
     // LDS: the bitonic exchange arrays, or (HBM path) the ranking tables
@@ -2113,7 +2117,7 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
             if (list) {
                 s_list[at] = (uint16_t)i;
             } else {
-                keys[base + at] = tkeys[i];
+                keys[base + at] = from[i];
                 vals[base + at] = i;
             }
             ++at;
@@ -2145,15 +2149,15 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
         const uint64_t* q = sc->quantiles ? quant + (uint64_t)blockIdx.x * kQuantiles : nullptr;
         bool slots = false;
         if (cnt <= kSlots / 4)
-            slots = bucket_sort_slots<1, GATHER>(tkeys, s_list, keys, vals, base, cnt, s_raw, q, ties);
+            slots = bucket_sort_slots<1, GATHER>(from, s_list, keys, vals, base, cnt, s_raw, q, ties);
         else if (cnt <= kSlots / 2)
-            slots = bucket_sort_slots<2, GATHER>(tkeys, s_list, keys, vals, base, cnt, s_raw, q, ties);
+            slots = bucket_sort_slots<2, GATHER>(from, s_list, keys, vals, base, cnt, s_raw, q, ties);
         else if (cnt <= kSlots)
-            slots = bucket_sort_slots<4, GATHER>(tkeys, s_list, keys, vals, base, cnt, s_raw, q, ties);
+            slots = bucket_sort_slots<4, GATHER>(from, s_list, keys, vals, base, cnt, s_raw, q, ties);
         if (GATHER && !slots && cnt <= kSlots) {
             // listed, but clustered: written out for the bitonic sort
             for (uint32_t i = tid; i < cnt; i += kBucketThreads) {
-                keys[base + i] = tkeys[s_list[i]];
+                keys[base + i] = from[s_list[i]];
                 vals[base + i] = s_list[i];
             }
         }
