@@ -901,20 +901,23 @@ __device__ __forceinline__ DeepKey deep_key(uint64_t key, double4 q, double E, i
     }
     return DeepKey{{w0, w1, w2}};
 }
+// The run headed at g, among the sorted keys [first, end): all of them, or one
+// bucket's, past which another block's keys are not sorted yet (and may still
+// be those of an earlier pass).
 template <int DIM>
-__device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t total,
+__device__ void order_tie_run(const SegDesc* __restrict__ desc, uint64_t first, uint64_t end,
                               const uint64_t* __restrict__ skeys, uint32_t* __restrict__ svals,
                               DeepKey* __restrict__ deep, uint32_t nseg, int segbits, int lmax,
                               uint64_t g) {
-    if (g + 1 >= total) return;
+    if (g + 1 >= end) return;
     const uint64_t key = skeys[g];
-    if (skeys[g + 1] != key || (g > 0 && skeys[g - 1] == key)) return;  // run heads only
+    if (skeys[g + 1] != key || (g > first && skeys[g - 1] == key)) return;  // run heads only
     const uint32_t s = seg_of_key(key, segbits);
     if (s >= nseg) return;
     const SegDesc& d = desc[s];
     uint64_t r = g + 1;
-    while (r + 1 < total && skeys[r + 1] == key && r + 1 - g < (uint64_t)kMaxTieRun) ++r;
-    if (r + 1 < total && skeys[r + 1] == key) {
+    while (r + 1 < end && skeys[r + 1] == key && r + 1 - g < (uint64_t)kMaxTieRun) ++r;
+    if (r + 1 < end && skeys[r + 1] == key) {
         atomicOr(&d.st->err, kErrDepth);
         return;
     }
@@ -949,7 +952,7 @@ __global__ __launch_bounds__(kBlock) void k_ties(const SegDesc* __restrict__ des
                                                  uint32_t* __restrict__ svals,
                                                  DeepKey* __restrict__ deep, uint32_t nseg,
                                                  int segbits, int lmax) {
-    order_tie_run<DIM>(desc, total, skeys, svals, deep, nseg, segbits, lmax,
+    order_tie_run<DIM>(desc, 0, total, skeys, svals, deep, nseg, segbits, lmax,
                        (uint64_t)blockIdx.x * kBlock + threadIdx.x);
 }
 
@@ -2234,7 +2237,8 @@ __global__ __launch_bounds__(kBucketThreads) __attribute__((amdgpu_waves_per_eu(
     }
     __syncthreads();
     for (uint32_t i = tid; i < cnt; i += kBucketThreads)
-        order_tie_run<DIM>(desc, total, keys, vals, deep, nseg, segbits, lmax, base + i);
+        order_tie_run<DIM>(desc, base, base + cnt, keys, vals, deep, nseg, segbits, lmax,
+                           base + i);
 }
 
 // Per sorted body: its common-prefix lengths with its neighbours give the

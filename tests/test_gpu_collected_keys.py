@@ -75,3 +75,30 @@ def test_buckets_past_the_cap_on_a_busy_gpu():
     for t in threads:
         t.join()
     assert all(g and all(g) for g in got)
+
+
+@pytest.mark.parametrize("cap", [0, 100, 4096])
+@pytest.mark.parametrize("n,run", [(900, 3), (3000, 2), (3000, 5), (9000, 30), (9000, 70),
+                                   (16384, 4), (16385, 4)])
+def test_runs_of_equal_keys_at_bucket_ends(n, run, cap):
+    """Bodies in runs of one cell of level 21 each, so that buckets begin and
+    end with a run; between passes some leave a run for one before or after
+    it, so that the previous pass's keys just past a bucket are its own first
+    or last key."""
+    rng = np.random.default_rng(n + run)
+    s = np.zeros(n, P.ENTITY)
+    cells = rng.choice(1 << 18, n // run + 1, replace=False)
+
+    def put(i, c):
+        for k, f in enumerate("xyz"):
+            s[f][i] = ((c >> (6 * k)) & 63) / 64.0 + 2e-7 + rng.uniform(0.0, 5e-7, len(i))
+
+    s["mass"] = rng.uniform(0.5, 1.5, n) / n
+    put(np.arange(n), np.repeat(cells, run)[:n])
+    s["x"][0] = -1.0  # (the extent: cells of level 21 are 2^-20 wide)
+    states = [s.copy()]
+    for _ in range(5):
+        some = rng.choice(np.arange(1, n), n // 8, replace=False)
+        put(some, rng.choice(cells, len(some)))
+        states.append(s.copy())
+    assert all(against_radix(states, cap))
