@@ -32,6 +32,8 @@ int pg_set_error(int code, const char* fmt, ...) {
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
     g_err = buf;
+    // (reported here: the check after the next launch must not find it)
+    if (code == PG_ERR_NOMEM) (void)hipGetLastError();
     return code;
 }
 
@@ -277,6 +279,14 @@ static void free_scratch(pg_engine* e) {
     e->scratch_bytes = 0;
     e->cap_bodies = e->cap_nodes = 0;
     e->cap_segs = e->cap_blocks = 0;
+    // nothing is left in it: where no new scratch follows (out of memory), an
+    // upload has no extents or tag to write and no tree is the last one built
+    e->sc = nullptr;
+    e->ext_partial = nullptr;
+    e->ext_valid = e->sorted_valid = 0;
+    e->ext_zero = 0;
+    e->last_sim = nullptr;
+    e->up_kind = -1;
 }
 
 extern "C" void pg_engine_destroy(pg_engine* e) {
