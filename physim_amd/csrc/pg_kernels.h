@@ -3449,7 +3449,8 @@ struct WalkConst {
 // close to call by t_yes and t_no or whose span does not advance: the caller
 // takes that step. (Every load is waited for inside; a mask written by a
 // vector compare is read by the scalar unit, or by a vector instruction at
-// least two instructions later.)
+// least two instructions later. M0, the lane of a writelane with two scalar
+// operands, is the compiler's to keep and no clobber names it: it is put back.)
 #define PG_WALK_RECORD(WHO, END, MASK)                                                          \
     "s_mov_b32 m0, %[items]\n\t"                                                                \
     END                                                                                         \
@@ -3529,6 +3530,7 @@ struct WalkConst {
     "s_cbranch_scc1 Lw" P "node%=\n\t"                                                          \
     "s_branch Lw" P "leaf%=\n"
 #define PG_WALK_LOOP(NEAR_A, NEAR_B)                                                            \
+    "s_mov_b32 %[keep], m0\n\t"                                                                 \
     "s_lshl_b32 %[st], %[k], 3\n\t"                                                             \
     "s_load_dwordx8 s[64:71], %[hot], %[st]\n\t"                                                \
     "s_load_dwordx2 s[72:73], %[span], %[k]\n"                                                  \
@@ -3537,7 +3539,8 @@ struct WalkConst {
     PG_WALK_SET("y", "x", "s[76:83]", "s[76:77]", "s[78:79]", "s[80:81]", "s82", "s83",         \
                 "s[84:85]", "s84", "s85", "s[64:71]", "s[72:73]", "s72", NEAR_B)                \
     "Lwend%=:\n\t"                                                                              \
-    "s_waitcnt lgkmcnt(0)\n\t"
+    "s_waitcnt lgkmcnt(0)\n\t"                                                                  \
+    "s_mov_b32 m0, %[keep]\n\t"
 // A node within the wave's level bounds: lanes whose own bounds hold its level
 // and that lie within extent 2^-level + margin of its centre on every axis
 // don't take it.
@@ -3564,15 +3567,15 @@ struct WalkConst {
 template <int DIM, bool NEAR>
 __device__ __forceinline__ void walk_items(WalkState& w, const WalkConst& c) {
     uint64_t act, m, m2;
-    uint32_t st, v0, v1;
+    uint32_t st, v0, v1, keep;
     double d0, d1, d2, q;
 #define PG_WALK_ASM(CODE, ...)                                                                  \
     asm volatile(CODE                                                                           \
                  : [b] "+&s"(w.b), [k] "+&s"(w.k8), [items] "+&s"(w.items), [leaf] "+&s"(w.leaf),   \
                    [it] "+&v"(w.it), [entry] "+&v"(w.entry), [skip] "+&v"(w.skip_until),           \
                    [act] "=&s"(act), [m] "=&s"(m), [m2] "=&s"(m2), [st] "=&s"(st),              \
-                   [v0] "=&v"(v0), [v1] "=&v"(v1), [d0] "=&v"(d0), [d1] "=&v"(d1),              \
-                   [d2] "=&v"(d2), [q] "=&v"(q)                                                 \
+                   [keep] "=&s"(keep), [v0] "=&v"(v0), [v1] "=&v"(v1), [d0] "=&v"(d0),          \
+                   [d1] "=&v"(d1), [d2] "=&v"(d2), [q] "=&v"(q)                                 \
                  : [hot] "s"(c.hot), [span] "s"(c.span), [bend] "s"(c.bend),                    \
                    [yes] "s"(c.t_yes), [no] "s"(c.t_no), [x] "v"(c.x), [y] "v"(c.y),            \
                    [z] "v"(c.z) __VA_ARGS__                                                     \
