@@ -3320,15 +3320,27 @@ __device__ __forceinline__ double refine_inverse(double x, double y) {
 // the six quotients and the compiler's square root took 110 (vector issue
 // bounds the FP64 sums: all pairs of 131,074 bodies 74.1 -> 43.6 ms, the walk of
 // 65,539 at theta 0.7 118 -> 102 us). The results are
-// the correctly rounded ones of those operations, as before. Squared
-// distances or masses far outside the range of either take the plain form.
+// the correctly rounded ones of those operations: with both bodies in pair_range
+// and the squared distance in (2^-600, 2^200), a component of the separation is
+// zero or at least 2^-353 (a difference of two doubles is a multiple of the
+// smaller one's last place), its quotient zero or at least 2^-453, and times the
+// masses at least 2^-813 and at most 2^400, so no quotient, residual or reciprocal
+// leaves the normal range. Anything else takes the plain form. (in_range: a and all
+// the sources that b is taken from are in pair_range, which is looked at once a
+// body, not once a pair.)
+constexpr double kPairMin = 0x1p-600, kPairMax = 0x1p+200;
+__device__ __forceinline__ bool pair_range(double x, double y, double z, double m) {
+    auto coord = [](double c) { return c == 0.0 || fabs(c) >= 0x1p-300; };
+    return coord(x) && coord(y) && coord(z) &&
+           (m == 0.0 || (fabs(m) >= 0x1p-180 && fabs(m) <= 0x1p+200));
+}
 __device__ __forceinline__ void pair_fp64(double ax, double ay, double az, double am, double bx,
-                                          double by, double bz, double bm, double e, double f[3]) {
+                                          double by, double bz, double bm, double e, bool in_range,
+                                          double f[3]) {
     const double d0 = ax - bx, d1 = ay - by, d2 = az - bz;
     const double s = d0 * d0 + d1 * d1 + d2 * d2;
     const double re = s + e;
-    if (__builtin_expect(s > 0x1p-700 && re < 0x1p+700 && fabs(am) < 0x1p+300 &&
-                             fabs(bm) < 0x1p+300, true)) {
+    if (__builtin_expect(in_range && s > kPairMin && re < kPairMax, true)) {
         const double y = __builtin_amdgcn_rsq(s);
         double g = s * y, h = 0.5 * y;  // towards sqrt(s) and 1 / (2 sqrt(s))
         const double r = fma(-h, g, 0.5);
@@ -3670,6 +3682,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     const double x = p.x, y = p.y, z = p.z, m = p.w;
     const bool fixed = !valid || tag_fixed(pr.w);
     bool history = true;  // the Stormer history holds (a step after the first)
+    const bool self_range = FP64 && pair_range(x, y, z, m);
     uint32_t* list = s_list[wv] + lane * kWalkStride;
     Kahan3 ka;
     ka.zero();
@@ -3787,6 +3800,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
             // in order
             const uint32_t cnt = w.entry - entry0;
             if (COUNT) count += cnt;
+            bool in_range = true;  // FP64: this lane's source is
             if (lane < w.items) {
                 const double4 q = gload((w.leaf >> lane) & 1ull
                                             ? leafpos + w.it
@@ -3794,7 +3808,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
                 s_src[wv][lane] = make_double2(q.x, q.y);
                 s_src[wv][kWalkItems + lane] =
                     make_double2(q.z, FP64 ? q.w : bits_f64((uint64_t)f32_bits((float)q.w)));
+                if (FP64) in_range = pair_range(q.x, q.y, q.z, q.w);
             }
+            const bool all_range = FP64 && self_range && !lanes_where(!in_range);
             wave_lds_sync();
             for (uint32_t t = 0; lanes_where(t < cnt); t += 4u) {
                 const uint32_t q = list[t >> 2];
@@ -3806,7 +3822,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
                         const uint32_t i = (q >> (8u * u)) & (kWalkItems - 1u);
                         const double2 a = s_src[wv][i], c = s_src[wv][kWalkItems + i];
                         if (t + u < cnt)
-                            pair_fp64(x, y, z, m, a.x, a.y, c.x, c.y, e, f64);
+                            pair_fp64(x, y, z, m, a.x, a.y, c.x, c.y, e, all_range, f64);
                     }
                 } else {
                     float3 v[4];
@@ -4038,21 +4054,25 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
     Kahan3 ka;
     ka.zero();
     double f64[3] = {0.0, 0.0, 0.0};
+    const bool self_range = FP64 && pair_range(x, y, z, m);
     for (uint64_t t0 = j0; t0 < j1; t0 += kBlock) {
         const uint64_t jj = t0 + threadIdx.x;
+        bool in_range = true;  // FP64: this thread's source is
         // mixed precision stages the mass as FP32 in the fourth word
         if (jj < j1) {
             const double4 p = d.spos[jj];
             sj[threadIdx.x] =
                 make_double4(p.x, p.y, p.z, FP64 ? p.w : bits_f64((uint64_t)f32_bits((float)p.w)));
+            if (FP64) in_range = pair_range(p.x, p.y, p.z, p.w);
         }
-        __syncthreads();
+        const bool tile_range = FP64 ? __syncthreads_and(in_range) != 0 : (__syncthreads(), true);
         const int cnt = (int)min((uint64_t)kBlock, j1 - t0);
         if (FP64) {
+            const bool all_range = self_range && tile_range;
 #pragma unroll 4
             for (int k = 0; k < cnt; ++k) {
                 const double4 b = sj[k];
-                pair_fp64(x, y, z, m, b.x, b.y, b.z, b.w, e, f64);
+                pair_fp64(x, y, z, m, b.x, b.y, b.z, b.w, e, all_range, f64);
             }
         } else {
             float px = 0.0f, py = 0.0f, pz = 0.0f;

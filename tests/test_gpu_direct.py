@@ -93,3 +93,51 @@ def test_energy_groups(engine, n):
                     [float((s["mass"] * speed).sum())] * 3)
     assert (np.abs(got - ref[:6]) <= (n + 1000) * 2.0 ** -53 * size).all()
     sim.close()
+
+
+@pytest.mark.parametrize("ma,mb", [
+    (1e-150, 1e-150), (1.0, 1e-300), (1e-300, 1e10), (2.0 ** -181, 2.0 ** -179), (0.0, 1.0),
+    (2.0 ** 199, 2.0 ** 201), (2.0 ** 290, 2.0 ** 290), (1e-155, 3e-155)])
+@pytest.mark.parametrize("scale,tiny,e", [
+    (1.0, 0.0, 0.5), (1.0, 1e-295, 0.5), (1.0, 3e-310, 0.0), (1e-8, 2.0 ** -301, 1e-30),
+    (2.0 ** 99, 2.0 ** -300, 0.0), (2.0 ** 101, 0.0, 1.0), (2.0 ** -301, 0.0, 0.0),
+    (2.0 ** -299, 0.0, 0.0)])
+def test_one_term_at_the_ends_of_the_range(engine, ma, mb, scale, tiny, e):
+    """Masses, separations and single components of one near and past the ends
+    of the fast form's range: the oracle's bits (infinities and NaN where it
+    has them), in the direct sum, and in the walk where the two bodies are far
+    enough apart for a tree."""
+    rng = np.random.default_rng(7)
+    for k in range(24):
+        p = rng.uniform(0.5, 1.0, (2, 3)) * scale * [[-1.0], [1.0]]
+        if tiny or k % 3 == 0:
+            p[:, k % 3] = rng.uniform(-1.0, 1.0, 2) * tiny
+        s = bodies(p, [ma * rng.uniform(0.9, 1.1), mb * rng.uniform(0.9, 1.1)])
+        sim = P.Sim(engine, s, kind="simple_astro", precision="fp64", e=e)
+        np.testing.assert_array_equal(sim.accel(), O.simple_transform(s, e))
+        sim.close()
+        if 1e-8 <= scale <= 1.0:
+            ref, _, fault = O.bh_transform(s, 0.0, e)
+            assert fault == 0
+            sim = P.Sim(engine, s, kind="astro2", precision="fp64", theta=0.0, e=e)
+            np.testing.assert_array_equal(sim.accel(), ref)
+            sim.close()
+
+
+def test_range_is_looked_at_for_every_source(engine):
+    """One source outside the range among 700: the sum of each body's terms in
+    source order, as one block sums them (n 2^-53 of the terms' magnitudes)."""
+    rng = np.random.default_rng(11)
+    for at in (0, 255, 256, 699):
+        s = bodies(rng.uniform(-1.0, 1.0, (700, 3)) * 1e-100, np.full(700, 1e-200))
+        s["mass"][at] = 1e-60
+        s["x"][at] = 1e-120
+        sim = P.Sim(engine, s, kind="simple_astro", precision="fp64", e=1e-190)
+        a = sim.accel()
+        ref = O.simple_transform(s, 1e-190)
+        pos = np.stack([s["x"], s["y"], s["z"]], 1)
+        r2 = ((pos[:, None] - pos[None]) ** 2).sum(-1)
+        size = (s["mass"] / (r2 + 1e-190)).sum(1)
+        assert np.isfinite(ref).all()
+        assert (np.abs(a - ref).max(1) <= 700 * 2.0 ** -53 * size).all()
+        sim.close()
