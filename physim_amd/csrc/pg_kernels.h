@@ -3711,15 +3711,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
         // and s formed with fused multiply-adds and the reference's rounded
         // quotient are within a few 1e-16 of exact, so outside a band of
         // 1e-10 around the threshold one FP64 comparison decides; inside it
-        // (or where theta or E leave the range in which no step under- or
-        // overflows: thresholds of NaN) the reference's own square root and
-        // division do. 9 vector instructions, where an FP32 quotient with its
-        // band took 25.
+        // the reference's own square root and division do. 9 vector
+        // instructions, where an FP32 quotient with its band took 25. A
+        // threshold past 2^800 or below 2^-800 (a theta out of all
+        // proportion) is taken no further than that: what lies beyond it is
+        // decided, the rest left to the division, as everything is for an
+        // extent in which a step could under- or overflow (thresholds of
+        // NaN). No quotient is below a theta of zero or less.
         const double t0 = (E / theta) * (E / theta);
-        const bool plain = theta > 0.0 && E > 0x1p-900 && E < 0x1p+900 && t0 > 0x1p-800 &&
-                           t0 < 0x1p+800;
-        const double t_yes = scalar_f64(plain ? t0 * (1.0 + 1e-10) : __builtin_nan(""));
-        const double t_no = scalar_f64(plain ? t0 * (1.0 - 1e-10) : __builtin_nan(""));
+        const double hi = t0 * (1.0 + 1e-10), lo = t0 * (1.0 - 1e-10);
+        const bool plain = theta > 0.0 && E > 0x1p-900 && E < 0x1p+900;
+        const double rest = theta <= 0.0 ? __builtin_inf() : __builtin_nan("");
+        const double t_yes = scalar_f64(plain ? (hi > 0x1p-800 ? hi : 0x1p-800) : rest);
+        const double t_no = scalar_f64(plain ? (lo < 0x1p+800 ? lo : 0x1p+800) : rest);
         // near field (no reference counterpart; off at 0): a cell at the
         // scale of the body's own leaf cell (its level and the kNearLevels
         // below) is opened, never taken whole, when the body lies within

@@ -98,3 +98,33 @@ def test_fixed_waves_and_short_segments(engine):
     for sim, ref in zip(sims, alone):
         np.testing.assert_array_equal(sim.download(), ref)
         sim.close()
+
+
+@pytest.mark.parametrize("theta", [0.0, -0.0, -1e300, float("-inf"), 5e-324, 1e-121, 2e-121, 1e120,
+                                   1.7e120, 1e308, float("inf")])
+@pytest.mark.parametrize("kind", ["astro2", "astro"])
+def test_angles_around_the_last_thresholds(engine, kind, theta):
+    """Squared extent over angle about 2^800 and 2^-800, and past any double:
+    an extent of 0.5 to 1 over 1.5e-121 and over 6.7e120."""
+    s = cloud(150, 9)
+    for f in "xyz":
+        s[f] *= 0.75
+    check(engine, s, theta, kind=kind)
+
+
+def test_an_angle_of_zero_costs_no_more_than_a_tiny_one(engine):
+    """Both open every cell: the time of the walk, the better of a few passes
+    (a division for every test takes 1.6 times as long)."""
+    s = cloud(3000, 5)
+    best = {}
+    engine.set_profiling(True)
+    for theta in (1e-9, 0.0, -1.0, 1e-200):
+        sim = P.Sim(engine, s, theta=theta, e=0.1)
+        for _ in range(6):
+            engine.profile_reset()
+            sim.accel()
+            best[theta] = min(best.get(theta, 1e9), engine.profile()["walk"][0])
+        sim.close()
+    engine.set_profiling(False)
+    print(best)
+    assert max(best.values()) <= 1.5 * best[1e-9]
