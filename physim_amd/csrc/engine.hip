@@ -59,6 +59,13 @@ struct EventPair {
     hipEvent_t a, b;
 };
 
+// One launch of the direct sum: a run of the batch's target tiles.
+struct DirectRound {
+    uint32_t blk0 = 0, blk1 = 0;    // blocks
+    uint64_t body0 = 0, body1 = 0;  // targets
+    uint64_t line0 = 0, lines = 0;  // partial sums
+};
+
 struct pg_engine {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -174,7 +181,8 @@ struct pg_engine {
     // what earlier calls held allocates nothing on the host either
     std::vector<pg_sim*> h_sims;
     std::vector<uint32_t> h_chunk0, h_nchunk, h_tile0;
-    std::vector<uint64_t> h_part_off;
+    std::vector<uint64_t> h_part_line;
+    std::vector<DirectRound> h_rounds;
 };
 
 struct pg_sim {
@@ -231,16 +239,6 @@ static uint64_t nodes_bound(uint64_t n, int dim, int lmax) {
     (void)dim;
     (void)lmax;
     return n + (n * (uint64_t)(kMaxLcp + 1) + 1) / 2 + 1;
-}
-
-extern "C" uint64_t pg_sim_bytes(uint64_t n, int32_t kind) {
-    const int dim = key_dim(kind);
-    const uint64_t scratch =
-        kind == PG_KIND_DIRECT
-            ? n * 24
-            : n * (8 * 2 + 4 * 2 + 4 + 4 + 1 + 8 + 24) + nodes_bound(n, dim, key_lmax(dim, 0)) *
-                                                      sizeof(NodeHot);
-    return state_bytes(n) + scratch;
 }
 
 // --------------------------------------------------------------- engine
@@ -570,6 +568,16 @@ static int clear_scratch_status(pg_engine* e) {
     return PG_OK;
 }
 
+// What a scratch grown to hold these takes (all that it holds now is kept).
+static uint64_t grown_scratch(pg_engine* e, uint64_t& bodies, uint64_t& nodes, uint32_t& segs,
+                              uint32_t& blocks) {
+    bodies = std::max({bodies, e->cap_bodies, (uint64_t)1024});
+    nodes = std::max({nodes, e->cap_nodes, (uint64_t)1024});
+    segs = std::max({segs, e->cap_segs, 4u});
+    blocks = std::max({blocks, e->cap_blocks, 16u});
+    return carve_scratch(e, nullptr, bodies, nodes, segs, blocks);
+}
+
 // Grows the batch scratch to hold `bodies` bodies, `nodes` tree nodes, `segs`
 // segments and `blocks` direct-sum blocks. One allocation, carved in place.
 // An engine on a fixed scratch (the allocation-free path) never grows: a
@@ -584,15 +592,7 @@ static int ensure_scratch(pg_engine* e, uint64_t bodies, uint64_t nodes, uint32_
                             "batch exceeds the fixed scratch (%llu bodies, %llu nodes, %u blocks)",
                             (unsigned long long)e->cap_bodies, (unsigned long long)e->cap_nodes,
                             e->cap_blocks);
-    bodies = std::max<uint64_t>(bodies, e->cap_bodies);
-    nodes = std::max<uint64_t>(nodes, e->cap_nodes);
-    segs = std::max<uint32_t>(segs, e->cap_segs);
-    blocks = std::max<uint32_t>(blocks, e->cap_blocks);
-    bodies = std::max<uint64_t>(bodies, 1024);
-    segs = std::max<uint32_t>(segs, 4);
-    blocks = std::max<uint32_t>(blocks, 16);
-    nodes = std::max<uint64_t>(nodes, 1024);
-    const uint64_t total = carve_scratch(e, nullptr, bodies, nodes, segs, blocks);
+    const uint64_t total = grown_scratch(e, bodies, nodes, segs, blocks);
     if (e->sims_bytes + total > e->budget)
         return pg_set_error(PG_ERR_BUDGET, "scratch of %llu bytes exceeds the HBM budget",
                             (unsigned long long)total);
@@ -655,19 +655,21 @@ static void ev_collect(pg_engine* e) {
 // all, eight waves a SIMD; where at most four shared one, 1,000, 8,195 and
 // 32,770 bodies took 94, 700 and 6,910 us in FP64, 20, 199 and 2,690 now with
 // their shared divisions, and 22, 116 and 873 us in mixed precision, 21, 60 and
-// 862 now). The partial sums take
-// at most kDirectPartBytes, what the allocation-free transform's node array
-// holds. In mixed precision the compensated sums run over kMaxDirectSplit
-// ranges of tiles whatever the groups, so that every size keeps the sums it had
-// with one block per range; more groups than ranges write each tile's partial
-// sum, which fits up to 18,900 bodies. All follow from the segment's own size,
-// so a segment sums alike alone and in a batch.
+// 862 now). Groups past the four ranges are made only while a segment's partial
+// sums take no more than kDirectPartBytes. In mixed precision the compensated
+// sums run over kMaxDirectSplit ranges of tiles whatever the groups, so that
+// every size keeps the sums it had with one block per range; more groups than
+// ranges write each tile's partial sum, which fits up to 18,900 bodies. All
+// follow from the segment's own size, so a segment sums alike alone and in a
+// batch. What the batch's partial sums take together is bounded by
+// direct_lines: past that they are formed a run of target tiles at a time.
 constexpr uint32_t kMaxDirectSplit = 4;
 constexpr uint64_t kDirectPartBytes = 16ull << 20;
 struct DirectSplit {
     uint32_t ranges = 1, groups = 1;
     bool fine = false;
-    uint64_t parts = 0;  // partial sums (24 bytes each)
+    uint32_t tiles = 1;  // target tiles
+    uint32_t lines = 0;  // lines of partial sums per target tile
 };
 static DirectSplit direct_split(uint64_t n, bool fp64) {
     DirectSplit d;
@@ -684,8 +686,36 @@ static DirectSplit direct_split(uint64_t n, bool fp64) {
         d.groups = (uint32_t)std::min<uint64_t>({fill, tiles, 255});
         d.fine = true;
     }
-    if (d.groups > 1) d.parts = d.fine ? (tiles * n + 1) / 2 : d.groups * n;
+    d.tiles = (uint32_t)tiles;
+    if (d.groups > 1) d.lines = d.fine ? d.tiles : 2 * d.groups;
     return d;
+}
+
+// The fewest lines of partial sums a direct batch of `total` lines, at most
+// `most` to a target tile, runs with: one tile's, and four partial sums a body
+// (2 tiles in 33 at 8,195 bodies in FP64, 128 blocks a launch).
+static uint64_t least_lines(uint64_t bodies, uint64_t total, uint64_t most) {
+    return std::min(total, std::max(most, bodies * 96 / kPartLine));
+}
+static uint64_t nodes_of_lines(uint64_t lines) {  // the node array holds them
+    return (lines * kPartLine + sizeof(NodeHot) - 1) / sizeof(NodeHot);
+}
+
+extern "C" uint64_t pg_sim_bytes(uint64_t n, int32_t kind) {
+    const int dim = key_dim(kind);
+    if (kind == PG_KIND_DIRECT) {
+        uint64_t nodes = 0;
+        uint32_t blocks = 0;
+        for (bool fp64 : {false, true}) {
+            const DirectSplit d = direct_split(n, fp64);
+            nodes = std::max(nodes, nodes_of_lines(least_lines(n, (uint64_t)d.tiles * d.lines,
+                                                               d.lines)));
+            blocks = std::max(blocks, d.tiles * d.groups);
+        }
+        return state_bytes(n) + carve_scratch(nullptr, nullptr, n, nodes, 1, blocks);
+    }
+    return state_bytes(n) + n * (8 * 2 + 4 * 2 + 4 + 4 + 1 + 8 + 24) +
+           nodes_bound(n, dim, key_lmax(dim, 0)) * sizeof(NodeHot);
 }
 
 struct BatchPlan {
@@ -699,11 +729,59 @@ struct BatchPlan {
     uint32_t nblocks = 0;
     uint32_t nchunks = 0;
     uint32_t ntiles = 0;  // node tiles
-    uint32_t max_group = 1;  // direct sum: the most source groups of a segment
     bool integrate = true;
     bool near = false;   // some segment walks with a near field (the walk that tests for it)
     bool count = false;  // some segment counts interactions (the walk that counts)
 };
+
+// How many lines of partial sums a direct batch of `total` lines, at most `most`
+// to a target tile, is given room for: all, up to kDirectRoundBytes or what the
+// scratch holds already; where the engine's budget is tight, no more than
+// least_lines and a 64th of what it leaves free, and where that does not fit,
+// one tile's.
+constexpr uint64_t kDirectRoundBytes = 64ull << 20;
+static uint64_t direct_lines(pg_engine* e, const BatchPlan& bp, uint64_t total, uint64_t most) {
+    const uint64_t held = e->scratch ? e->cap_nodes * sizeof(NodeHot) / kPartLine : 0;
+    if (e->fixed_scratch) return std::min(total, held);
+    auto takes = [&](uint64_t lines) {
+        uint64_t bodies = bp.total, nodes = nodes_of_lines(lines);
+        uint32_t segs = bp.nseg, blocks = bp.nblocks;
+        return e->sims_bytes + grown_scratch(e, bodies, nodes, segs, blocks);
+    };
+    const uint64_t least = least_lines(bp.total, total, most);
+    uint64_t lines = std::max(least, std::min(total, kDirectRoundBytes / kPartLine));
+    if (lines > held) {
+        const uint64_t with = takes(least);
+        if (with > e->budget) lines = std::min(total, most);
+        else lines = std::min(lines, least + (e->budget - with) / 64 / kPartLine);
+    }
+    return std::max(lines, std::min(total, held));
+}
+
+// The launches of a direct batch whose partial sums have room for `room` lines.
+static void plan_rounds(pg_engine* e, const std::vector<pg_sim*>& sims, bool fp64, uint64_t room) {
+    e->h_rounds.clear();
+    DirectRound r;
+    uint64_t off = 0;
+    for (const pg_sim* s : sims) {
+        const DirectSplit ds = direct_split(s->n, fp64);
+        for (uint32_t t = 0; t < ds.tiles;) {
+            uint32_t k = ds.tiles - t;
+            if (ds.lines) k = (uint32_t)std::min<uint64_t>(k, (room - r.lines) / ds.lines);
+            if (k == 0) {  // (room for one tile at least)
+                e->h_rounds.push_back(r);
+                r = DirectRound{r.blk1, r.blk1, r.body1, r.body1, r.line0 + r.lines, 0};
+                continue;
+            }
+            t += k;
+            r.blk1 += k * ds.groups;
+            r.lines += (uint64_t)k * ds.lines;
+            r.body1 = off + std::min<uint64_t>(s->n, (uint64_t)t * kBlock);
+        }
+        off += s->n;
+    }
+    e->h_rounds.push_back(r);
+}
 
 static inline unsigned grid_for(uint64_t n, unsigned cap) {
     uint64_t g = (n + kBlock - 1) / kBlock;
@@ -916,15 +994,17 @@ static void enqueue_direct_step(pg_engine* e, const BatchPlan& bp, int q, bool c
     launch(e, cap, "prep", [&] {
         k_prep<<<1, kBlock, 0, st>>>(desc, bp.nseg, e->sc, INTEG ? 1 : 0);
     });
-    // (one timed bracket: the sum and, where sources are split, the pass
-    // that adds the partial sums and stores)
+    // (one timed bracket: the sums and, where sources are split, the passes
+    // that add the partial sums and store)
     launch(e, cap, "direct", [&] {
-        double* part = reinterpret_cast<double*>(e->hot);
-        k_direct<FP64, INTEG><<<bp.nblocks, kBlock, 0, st>>>(desc, e->blk_seg, e->blk_tile,
-                                                            part, e->acc_out);
-        if (bp.max_group > 1)
-            k_direct_finish<FP64, INTEG><<<grid_for(bp.total, 1u << 30), kBlock, 0, st>>>(
-                desc, e->seg_off, bp.nseg, bp.total, part, e->acc_out);
+        float* part = reinterpret_cast<float*>(e->hot);
+        for (const DirectRound& r : e->h_rounds) {
+            k_direct<FP64, INTEG><<<r.blk1 - r.blk0, kBlock, 0, st>>>(
+                desc, e->blk_seg + r.blk0, e->blk_tile + r.blk0, part, r.line0, e->acc_out);
+            if (r.lines)
+                k_direct_finish<FP64, INTEG><<<grid_for(r.body1 - r.body0, 1u << 30), kBlock, 0, st>>>(
+                    desc, e->seg_off, bp.nseg, r.body0, r.body1, part, r.line0, e->acc_out);
+        }
     });
 }
 
@@ -1273,28 +1353,29 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     if (nodes >= (1ull << 32)) return pg_set_error(PG_ERR_ARG, "tree too large for 32-bit nodes");
     e->h_blk_seg.clear();
     e->h_blk_tile.clear();
-    std::vector<uint64_t>& part_off = e->h_part_off;
-    part_off.assign(bp.nseg, 0ull);
+    std::vector<uint64_t>& part_line = e->h_part_line;
+    part_line.assign(bp.nseg, 0ull);
     if (bp.kind == PG_KIND_DIRECT) {
         // Blocks: per segment, target tile and source group (group in the
-        // tile word's top 8 bits). A segment's partial sums live in the node
-        // array, which the direct sum does not otherwise use.
-        uint64_t part = 0;
+        // tile word's top 8 bits). The partial sums live in the node array,
+        // which the direct sum does not otherwise use.
+        uint64_t lines = 0, most = 0;
         for (uint32_t s = 0; s < bp.nseg; ++s) {
-            const uint32_t nb = (uint32_t)((sims[s]->n + kBlock - 1) / kBlock);
             const DirectSplit ds = direct_split(sims[s]->n, bp.precision == PG_PREC_FP64);
-            for (uint32_t t = 0; t < nb; ++t)
+            for (uint32_t t = 0; t < ds.tiles; ++t)
                 for (uint32_t p = 0; p < ds.groups; ++p) {
                     e->h_blk_seg.push_back(s);
                     e->h_blk_tile.push_back(t | (p << 24));
                 }
-            part_off[s] = part;
-            part += ds.parts;
-            bp.max_group = std::max(bp.max_group, ds.groups);
+            part_line[s] = lines;
+            lines += (uint64_t)ds.tiles * ds.lines;
+            most = std::max<uint64_t>(most, ds.lines);
         }
         bp.nblocks = (uint32_t)e->h_blk_seg.size();
-        nodes = (part * 24 + sizeof(NodeHot) - 1) / sizeof(NodeHot);
-        if (nodes >= (1ull << 32)) return pg_set_error(PG_ERR_ARG, "direct-sum partials too large");
+        const uint64_t room = direct_lines(e, bp, lines, most);
+        if (room < most) return pg_set_error(PG_ERR_INTERNAL, "no room for a tile's partial sums");
+        nodes = nodes_of_lines(room);
+        plan_rounds(e, sims, bp.precision == PG_PREC_FP64, room);
     }
     e->h_ext_seg.clear();
     e->h_ext_chunk.clear();
@@ -1369,7 +1450,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
             d.nsplit = ds.ranges;
             d.ngroup = ds.groups;
             d.fine = ds.fine ? 1u : 0u;
-            d.part_off = part_off[s];
+            d.part_line = part_line[s];
             d.near = sm->near;
         }
         off += sm->n;
@@ -2201,6 +2282,8 @@ static int noalloc_setup(NoAllocCtx& c, int device, hipStream_t stream) {
     // (ceil(n / 256) target tiles times at most 2^19 / n + 1 blocks, 255 of a
     // tile's and no more than it has groups of kDirectUnit sources)
     const uint32_t blocks = (1u << 19) / kBlock + 4 * (uint32_t)((n + kBlock - 1) / kBlock);
+    // (the node array holds a segment's partial sums in one round, or in two
+    // where whole tiles of 256 make them a little more)
     static_assert(kNoAllocMaxBodies * kNoAllocNodesPerBody * sizeof(NodeHot) >= kDirectPartBytes,
                   "the direct sum's partial sums in the node array");
     pg_engine& e = c.eng;
@@ -2221,7 +2304,8 @@ static int noalloc_setup(NoAllocCtx& c, int device, hipStream_t stream) {
     PG_TRY(clear_scratch_status(&e));
     const uint64_t chunks = n / kExtentChunk + 2, tiles = n / kNodeTile + 2;
     e.h_sims.reserve(1);
-    e.h_part_off.reserve(1);
+    e.h_part_line.reserve(1);
+    e.h_rounds.reserve(4);
     e.h_chunk0.reserve(1);
     e.h_nchunk.reserve(1);
     e.h_tile0.reserve(1);

@@ -53,6 +53,11 @@ constexpr int kMaxTieRun = 256;    // longest run of equal keys ordered by their
 constexpr int kMaxLcp = 64;        // deepest common prefix, in levels, of two bodies: the
                                    // reference recurses to depth 64 (octree.rs:60-62)
 constexpr int kDirectUnit = 32;    // sources per group of the FP64 direct sum: a multiple of this
+// A line of the direct sum's partial sums: those of a target tile's bodies over
+// one source tile (mixed precision, FP32), or half of those over one group (FP64
+// words, two lines). A target tile's lines lie together, the tiles in batch order.
+constexpr int kPartFloats = 3 * kBlock;
+constexpr uint64_t kPartLine = kPartFloats * sizeof(float);
 constexpr int kDeepWords = 3;      // words of a tied body's deep key
 static_assert(kMaxLcp + 1 == kTopSlots, "every level of an internal node has its slot");
 
@@ -113,7 +118,7 @@ struct SegDesc {
     uint32_t nsplit;  // direct sum, mixed precision: ranges of source tiles summed apart
     uint32_t ngroup;  // direct sum: blocks summing one target tile, each over a group of source tiles
     uint32_t fine;    // mixed precision: more groups than ranges (every tile's partial sum is kept)
-    uint64_t part_off;  // direct sum with ngroup > 1: first partial sum (x3 doubles) of the segment
+    uint64_t part_line;  // direct sum with ngroup > 1: the segment's first line of partial sums
     double near;      // near field in widths of the body's own leaf cell (0: off)
 };
 

@@ -4026,18 +4026,19 @@ __device__ __forceinline__ void direct_store(const SegDesc& d, uint64_t i, doubl
 // partial into a compensated FP32 sum over one of d.nsplit ranges of tiles;
 // with more groups than ranges (d.fine) each tile's partial is written out and
 // k_direct_finish forms the same compensated sums. Reads src, writes dst (same
-// order).
+// order). A launch takes the blocks of a run of the batch's target tiles, whose
+// partial sums are lines line0 and on of all the batch's, from `part`.
 template <bool FP64, bool INTEGRATE>
 __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ desc,
                                                    const uint32_t* __restrict__ blk_seg,
                                                    const uint32_t* __restrict__ blk_tile,
-                                                   double* __restrict__ part,
+                                                   float* __restrict__ part, uint64_t line0,
                                                    double* __restrict__ acc_out) {
     __shared__ double4 sj[kBlock];
     const uint32_t s = blk_seg[blockIdx.x];
     const SegDesc& d = desc[s];
     const uint32_t tw = blk_tile[blockIdx.x];
-    const uint64_t i = (uint64_t)(tw & 0xFFFFFFu) * kBlock + threadIdx.x;
+    const uint64_t tile = tw & 0xFFFFFFu, i = tile * kBlock + threadIdx.x;
     const uint32_t sp = tw >> 24, ng = d.ngroup;
     const bool fine = !FP64 && d.fine != 0;
     constexpr uint64_t kUnit = FP64 ? kDirectUnit : kBlock;
@@ -4100,8 +4101,9 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
             }
             if (fine) {
                 if (valid) {
-                    float* o = reinterpret_cast<float*>(part + 3 * d.part_off) +
-                               3 * (t0 / kBlock * d.n + i);
+                    float* o = part +
+                               (d.part_line + tile * units + t0 / kBlock - line0) * kPartFloats +
+                               3 * threadIdx.x;
                     o[0] = px; o[1] = py; o[2] = pz;
                 }
             } else {
@@ -4120,39 +4122,42 @@ __global__ __launch_bounds__(kBlock) void k_direct(const SegDesc* __restrict__ d
         fz = (double)ka.sz - (double)ka.cz;
     }
     if (ng > 1) {
-        double* o = part + 3 * (d.part_off + (uint64_t)sp * d.n + i);
+        double* o = reinterpret_cast<double*>(
+                        part + (d.part_line + 2 * (tile * ng + sp) - line0) * kPartFloats) +
+                    3 * threadIdx.x;
         o[0] = fx; o[1] = fy; o[2] = fz;
         return;
     }
     direct_store<FP64, INTEGRATE>(d, i, x, y, z, m, fixed, fx, fy, fz, acc_out);
 }
 
-// Bodies of segments whose sources k_direct split: the partial sums added in
-// group order (or, d.fine, the tiles' compensated sums of each range, added in
+// Bodies [g0, g1) of the batch, the targets of one launch of k_direct, where
+// their segment's sources were split: the partial sums added in group order (or, d.fine, the tiles' compensated sums of each range, added in
 // range order), then the store.
 template <bool FP64, bool INTEGRATE>
 __global__ __launch_bounds__(kBlock) void k_direct_finish(const SegDesc* __restrict__ desc,
                                                           const uint64_t* __restrict__ seg_off,
-                                                          uint32_t nseg, uint64_t total,
-                                                          const double* __restrict__ part,
+                                                          uint32_t nseg, uint64_t g0, uint64_t g1,
+                                                          const float* __restrict__ part,
+                                                          uint64_t line0,
                                                           double* __restrict__ acc_out) {
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= total) return;
+    const uint64_t g = g0 + (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (g >= g1) return;
     const SegDesc& d = desc[seg_of(seg_off, nseg, g)];
     const uint32_t ng = d.ngroup;
     if (ng <= 1) return;
-    const uint64_t i = g - d.off;
+    const uint64_t i = g - d.off, tile = i / kBlock, l = i % kBlock;
     double fx = 0.0, fy = 0.0, fz = 0.0;
     if (!FP64 && d.fine) {
         const uint64_t tiles = (d.n + kBlock - 1) / kBlock;
-        const float* o = reinterpret_cast<const float*>(part + 3 * d.part_off) + 3 * i;
+        const float* o = part + (d.part_line + tile * tiles - line0) * kPartFloats + 3 * l;
         for (uint32_t sp = 0; sp < d.nsplit; ++sp) {
             Kahan3 ka;
             ka.zero();
             const uint64_t t1 = tiles * (sp + 1) / d.nsplit;
 #pragma unroll 4
             for (uint64_t t = tiles * sp / d.nsplit; t < t1; ++t) {
-                const float* v = o + 3 * t * d.n;
+                const float* v = o + t * kPartFloats;
                 ka.add(v[0], v[1], v[2]);
             }
             fx += (double)ka.sx - (double)ka.cx;
@@ -4160,9 +4165,12 @@ __global__ __launch_bounds__(kBlock) void k_direct_finish(const SegDesc* __restr
             fz += (double)ka.sz - (double)ka.cz;
         }
     } else {
+        const double* first = reinterpret_cast<const double*>(
+                                  part + (d.part_line + 2 * tile * ng - line0) * kPartFloats) +
+                              3 * l;
 #pragma unroll 4
         for (uint32_t sp = 0; sp < ng; ++sp) {
-            const double* o = part + 3 * (d.part_off + (uint64_t)sp * d.n + i);
+            const double* o = first + (uint64_t)sp * kPartFloats;
             fx += o[0]; fy += o[1]; fz += o[2];
         }
     }
