@@ -758,6 +758,32 @@ static uint64_t direct_lines(pg_engine* e, const BatchPlan& bp, uint64_t total, 
     return std::max(lines, std::min(total, held));
 }
 
+void pg_group_add(pg_group_need* g, uint64_t n) {
+    if (!n) return;
+    g->bodies += n;
+    g->segs += 1;
+    if (g->kind != PG_KIND_DIRECT) return;
+    const DirectSplit d = direct_split(n, g->precision == PG_PREC_FP64);
+    g->blocks += d.tiles * d.groups;
+    g->lines += (uint64_t)d.tiles * d.lines;
+    g->most = std::max<uint64_t>(g->most, d.lines);
+}
+
+uint64_t pg_engine_bytes_with(pg_engine* e, const pg_group_need* groups, size_t count, uint64_t n) {
+    std::lock_guard<std::recursive_mutex> lk(e->mu);
+    uint64_t bodies = 0, nodes = 0;
+    uint32_t segs = 0, blocks = 0;
+    for (const pg_group_need* g = groups; g != groups + count; ++g) {
+        bodies = std::max(bodies, g->bodies);
+        segs = std::max(segs, g->segs);
+        blocks = std::max(blocks, g->blocks);
+        nodes = std::max(nodes, g->kind == PG_KIND_DIRECT
+                                    ? nodes_of_lines(least_lines(g->bodies, g->lines, g->most))
+                                    : nodes_bound(g->bodies, key_dim(g->kind), 0) + g->segs);
+    }
+    return e->sims_bytes + state_bytes(n) + grown_scratch(e, bodies, nodes, segs, blocks);
+}
+
 // The launches of a direct batch whose partial sums have room for `room` lines.
 static void plan_rounds(pg_engine* e, const std::vector<pg_sim*>& sims, bool fp64, uint64_t room) {
     e->h_rounds.clear();

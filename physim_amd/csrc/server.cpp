@@ -104,30 +104,42 @@ extern "C" int pg_server_tick(pg_server* s, uint32_t max_steps, uint32_t* n_acti
     if (!s) return pg_set_error(PG_ERR_ARG, "server is NULL");
     std::lock_guard<std::mutex> lk(s->mu);
     if (max_steps == 0) max_steps = 1;
-    // admission, in arrival order
+    // admission, in arrival order: a request waits while its state and the
+    // scratch of all that would then be stepped do not fit the budget
+    auto group_of = [](const Request* r) { return r->params.kind * 4 + r->params.precision; };
+    std::map<int, pg_group_need> needs;
+    auto add = [&](const Request* r) {
+        pg_group_need& g = needs[group_of(r)];
+        g.kind = r->params.kind;
+        g.precision = r->params.precision;
+        pg_group_add(&g, r->state.size());
+    };
+    for (const Request* r : s->active) add(r);
     while (!s->queue.empty() && (s->max_active == 0 || s->active.size() < s->max_active)) {
         Request* r = s->queue.front();
         uint64_t used = 0, budget = 0;
         pg_engine_memory(s->eng, &used, &budget);
-        const uint64_t need = pg_sim_bytes(r->state.size(), r->params.kind);
-        if (!s->active.empty() && used + need > budget) break;  // wait for memory
+        const std::map<int, pg_group_need> without = needs;
+        add(r);
+        std::vector<pg_group_need> with;
+        for (auto& kv : needs) with.push_back(kv.second);
+        if (!s->active.empty() &&
+            pg_engine_bytes_with(s->eng, with.data(), with.size(), r->state.size()) > budget)
+            break;  // wait for memory
         s->queue.pop_front();
         r->info.admit_s = s->now();
         int rc = pg_sim_create(s->eng, r->state.size(), &r->params, &r->sim);
         if (rc == PG_OK) rc = pg_sim_upload(r->sim, r->state.data(), r->state.size());
-        if (rc != PG_OK) {
+        if (rc != PG_OK || r->remaining == 0) {
             finish(s, r, (uint32_t)rc);
-            continue;
-        }
-        if (r->remaining == 0) {
-            finish(s, r, PG_OK);
+            needs = without;
             continue;
         }
         s->active.push_back(r);
     }
     // co-batched steps per (kind, precision) group
     std::map<int, std::vector<Request*>> groups;
-    for (Request* r : s->active) groups[r->params.kind * 4 + r->params.precision].push_back(r);
+    for (Request* r : s->active) groups[group_of(r)].push_back(r);
     for (auto& kv : groups) {
         std::vector<Request*>& g = kv.second;
         uint32_t k = max_steps;
