@@ -99,7 +99,9 @@ int pg_engine_set_sort(pg_engine* eng, uint32_t max_buckets, uint32_t bucket_cap
  * reference counterpart. */
 typedef struct pg_tuning {
     uint32_t max_buckets;   /* sample sort up to this many buckets (<= 8192; 0: radix sort) */
-    uint32_t bucket_keys;   /* mean keys per sample-sort bucket (256..4096; default 1664) */
+    uint32_t bucket_keys;   /* mean keys per sample-sort bucket (256..4096); 1664, the default,
+                               stands for 384 in batches of up to 131,072 bodies, 1,024 up to
+                               524,288 and 1,664 past them; any other is used as it is */
     uint32_t walk_run_log2; /* the walk's blocks go to each XCD in runs of 2^this (default 4) */
     uint32_t lds_buckets;   /* up to this many buckets every key tile holds the splitters in
                                LDS; more: in HBM behind a coarse table (<= 1024; 0: 1024) */

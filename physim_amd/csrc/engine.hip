@@ -99,7 +99,7 @@ struct pg_engine {
     uint32_t* bbase = nullptr;     // sample sort: first key of each bucket
     uint32_t max_buckets = kMaxWideBuckets;  // larger batches use the radix sort
     uint32_t lds_buckets = kMaxBuckets;  // more buckets: splitters in HBM (coarse table in LDS)
-    uint32_t bucket_keys = kBucketKeys;  // keys per sample-sort bucket (mean)
+    uint32_t bucket_keys = kBucketKeys;  // keys per sample-sort bucket (mean; the default: mean_bucket)
     uint32_t walk_run_log2 = 4;          // walk blocks per XCD run: 2^walk_run_log2
     uint64_t ext_valid = 0;  // batch whose extent partials the last step left (0: none)
     uint32_t ext_zero = 0;   // partials from the first that are known to be zero
@@ -815,6 +815,13 @@ static inline unsigned grid_for(uint64_t n, unsigned cap) {
     return (unsigned)std::min<uint64_t>(g, cap);
 }
 
+// Mean keys of a bucket for a batch of `total` bodies: by its size, unless a
+// tuning names another than the default.
+static uint64_t mean_bucket(const pg_engine* e, uint64_t total) {
+    if (e->bucket_keys != (uint32_t)kBucketKeys) return e->bucket_keys;
+    return total <= kFewBodies ? kBucketKeysFew : total <= kMoreBodies ? kBucketKeysMore : kBucketKeys;
+}
+
 // How many lanes of a wave walk a body, as a power of two. A wave's time is
 // the items of all its bodies, and a small batch leaves the chip short of
 // waves (1,024 SIMDs): fewer bodies to a wave are more and shorter walks, up
@@ -1365,11 +1372,7 @@ static int run_batch(pg_engine* e, pg_sim* const* sims_in, uint32_t count, uint3
     {
         // a batch past max_buckets of bucket_keys grows its buckets up to
         // the slot sort's reach (kSlots keys) before it takes the radix sort
-        uint64_t keys_per = e->bucket_keys;
-        if (bp.total <= kFewBodies)
-            keys_per = std::min<uint64_t>(keys_per, kBucketKeysFew);
-        else if (bp.total <= kMoreBodies)
-            keys_per = std::min<uint64_t>(keys_per, kBucketKeysMore);
+        uint64_t keys_per = mean_bucket(e, bp.total);
         if (e->max_buckets && (bp.total + keys_per - 1) / keys_per > e->max_buckets)
             keys_per = std::max<uint64_t>(keys_per, (bp.total + e->max_buckets - 1) / e->max_buckets);
         const uint64_t nb = (bp.total + keys_per - 1) / keys_per;
@@ -1921,7 +1924,8 @@ extern "C" int pg_engine_autotune(pg_engine* e, pg_sim* const* sims, uint32_t co
                                       : std::vector<uint32_t>{e->walk_run_log2};
     std::vector<std::pair<uint32_t, uint32_t>> sorts;  // (max_buckets, bucket_keys)
     if (tree) {
-        for (uint32_t bk : {1280u, 1664u, 2048u})
+        // (the default, 1664, is 384 or 1024 in a smaller batch: mean_bucket)
+        for (uint32_t bk : {1280u, (uint32_t)kBucketKeys, 2048u})
             if ((total + bk - 1) / bk <= (uint64_t)kMaxWideBuckets)
                 sorts.push_back({kMaxWideBuckets, bk});
         sorts.push_back({0u, kBucketKeys});
