@@ -84,7 +84,9 @@ void pg_engine_destroy(pg_engine* eng);
 /* Bytes of device memory the engine holds / its budget. */
 int pg_engine_memory(pg_engine* eng, uint64_t* used, uint64_t* budget);
 /* Device memory a simulation of n bodies needs (state + its share of
- * scratch), used for admission against the budget. */
+ * scratch), for planning against the budget. For the direct sum the scratch
+ * that a pass runs with (it takes up to 64 MB more where the budget leaves
+ * them free); the server counts the scratch of all that it steps together. */
 uint64_t pg_sim_bytes(uint64_t n, int32_t kind);
 /* Capture repeated steps in hipGraphs (default on). */
 int pg_engine_set_graphs(pg_engine* eng, int enable);

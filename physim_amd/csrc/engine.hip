@@ -659,7 +659,7 @@ static void ev_collect(pg_engine* e) {
 // sums take no more than kDirectPartBytes. In mixed precision the compensated
 // sums run over kMaxDirectSplit ranges of tiles whatever the groups, so that
 // every size keeps the sums it had with one block per range; more groups than
-// ranges write each tile's partial sum, which fits up to 18,900 bodies. All
+// ranges write each tile's partial sum, which fits up to 18,893 bodies. All
 // follow from the segment's own size, so a segment sums alike alone and in a
 // batch. What the batch's partial sums take together is bounded by
 // direct_lines: past that they are formed a run of target tiles at a time.

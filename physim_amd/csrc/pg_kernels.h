@@ -3318,8 +3318,8 @@ __device__ __forceinline__ double refine_inverse(double x, double y) {
 // also leaves the root's reciprocal), two reciprocals and three operations a
 // quotient, 60 vector instructions, where a division of its own for each of
 // the six quotients and the compiler's square root took 110 (vector issue
-// bounds the FP64 sums: all pairs of 131,074 bodies 74.1 -> 43.6 ms, the walk of
-// 65,539 at theta 0.7 118 -> 102 us). The results are
+// bounds the FP64 sums: all pairs of 131,074 bodies 71.4 -> 43.0 ms, the walk of
+// 65,539 at theta 0.7 118 -> 104 us). The results are
 // the correctly rounded ones of those operations: with both bodies in pair_range
 // and the squared distance in (2^-600, 2^200), a component of the separation is
 // zero or at least 2^-353 (a difference of two doubles is a multiple of the
@@ -3389,8 +3389,9 @@ __device__ __forceinline__ void pair_fp64(double ax, double ay, double az, doubl
 // 128, 3% fewer terms but half the waves. Against the walk with one phase (a
 // term per item, six selects to keep it): 262,144-body Plummer sphere at theta
 // 0.5 645 -> 390 us, 1M-body collision with a near field 2470 -> 1550,
-// 65,539-body cube at theta 0.7 in FP64 193 -> 118, 1M-body cube at theta 1.5
-// (one or two items a wave) 41.4 and 41.5.
+// 65,539-body cube at theta 0.7 in FP64 193 -> 118. At theta 1.5 (one or two items
+// a wave) there is nothing to gain, and the lists in LDS leave six waves a SIMD
+// where eight were resident: 1M-body cube 33.4 -> 35.1.
 constexpr uint32_t kWalkItems = 64;  // items per chunk: one source fetch per lane
 constexpr uint32_t kWalkStride = 17; // words per lane's list of byte entries: an odd LDS stride
 static_assert(kWalkItems == 64 && 4 * kWalkStride > kWalkItems && kWalkStride % 2 == 1,

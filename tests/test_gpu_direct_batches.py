@@ -74,3 +74,12 @@ def test_batch_in_a_tight_budget(engine, precision):
         eng.batch_step(sims, 5)
         for sim, s in zip(sims, states):
             assert sim.download().tobytes() == alone(engine, s, 5, **kw)[0]
+
+
+@pytest.mark.parametrize("n", [18688, 18689, 18893, 18894])
+def test_allocation_free_in_two_rounds(engine, n):
+    """Its node array holds 5,461 lines of partial sums: 73 x 73 tiles, not 74 x 74."""
+    s = bodies(n, n)
+    kw = dict(kind="simple_astro", precision="mixed", e=0.1)
+    for _ in range(2):
+        assert engine.transform_noalloc(s, **kw).tobytes() == engine.transform(s, **kw).tobytes()
